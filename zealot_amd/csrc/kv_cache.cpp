@@ -1265,7 +1265,9 @@ int decode_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState 
     // layer's pools, q or scales: the layers of one step share it.
     const uintptr_t hdr[] = {(uintptr_t)n,          (uintptr_t)num_heads,     stride,
                              (uintptr_t)nsg,        (uintptr_t)sp.total_pages, (uintptr_t)c->d_ws.p,
-                             (uintptr_t)c->d_ws.cap, (uintptr_t)c->tbl_version, (uintptr_t)max_waves};
+                             (uintptr_t)c->d_ws.cap, (uintptr_t)c->tbl_version, (uintptr_t)max_waves,
+                             // f32: operands that are not 16-byte aligned take a path without a plan
+                             c->dtype == ZK_F32 ? ((uintptr_t)q | (uintptr_t)out | (uintptr_t)(q_stride * 4)) & 15u : 0u};
     std::vector<char> sig((const char *)hdr, (const char *)hdr + sizeof(hdr));
     sig.insert(sig.end(), host.data(), host.data() + len_bytes);
     sig.insert(sig.end(), host.data() + len_bytes + sc_bytes, host.data() + len_bytes + sc_bytes + share_bytes);

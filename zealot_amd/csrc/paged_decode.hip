@@ -15,12 +15,15 @@
 //                     entry that is < 0 or >= num_blocks (paged_attention.cu:66-67)
 //   plan_kernel       partitions -> work-item descriptors, longest first;
 //                     resets the queue
-//   decode_mfma_kernel  bf16 / fp8 pools, D in {64,128}, G in {1,2,4,8}:
+//   decode_mfma_kernel  bf16 / fp8 / f32 pools, D in {64,128}, G in {1,2,4,8}:
 //       persistent one-wave workgroups take (sequence or subgroup, partition,
 //       kv-head) items from an atomic queue (no tail of short waves), stream
 //       each page through LDS with global_load_lds, and run QK^T and PV on
 //       MFMA with a lazily rescaled softmax (details at the kernel).
-//   decode_generic_kernel  any dtype / D <= 256 / G <= 16 (fp32 pools):
+//       Small and mid-sized batches run it without plan and queue (DIRECT): one
+//       workgroup per (kv-head, partition, sequence).  f32 pools use the f32
+//       MFMA (no precision is given up).
+//   decode_generic_kernel  any dtype / D <= 256 / G <= 16:
 //       one wavefront per (partition, kv-head, sequence); token-per-lane QK on
 //       the VALU, readlane-broadcast PV.
 //   decode_reduce_kernel  log-sum-exp merge of the partitions.
@@ -28,10 +31,12 @@
 // scale * log2(e) and exponentiated with exp2 (the FlashAttention trick).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <string>
+#include <type_traits>
 #include <utility>
 
 #include "zk_common.h"
@@ -161,8 +166,11 @@ __device__ __forceinline__ int shared_parts_of(const Params &p, int n) {
     return pb > 0 ? (pb + p.shared_part_pages - 1) / p.shared_part_pages : 0;
 }
 // Partitions of the pages after the shared prefix (the sequence's own items).
+// PLANLESS launches have no eff_len: the length is the caller's.
+template <bool PLANLESS = false>
 __device__ __forceinline__ int private_parts_of(const Params &p, int n) {
-    const int pages = (p.eff_len[n] + p.block_size - 1) / p.block_size;
+    const int len = PLANLESS ? min(max(p.seq_lens[n], 0), p.max_blocks * p.block_size) : p.eff_len[n];
+    const int pages = (len + p.block_size - 1) / p.block_size;
     const int rest = pages - prefix_pages_of(p, n);
     return rest > 0 ? (rest + p.part_pages - 1) / p.part_pages : 0;
 }
@@ -241,6 +249,10 @@ constexpr int kDescPages = 4;
 #define ZK_DECODE_STAGES 2
 #endif
 constexpr int kStages = ZK_DECODE_STAGES;
+
+// Planless launches (DIRECT): most pages of a partition (one table entry per
+// lane).
+constexpr int kDirectPages = 64;
 
 __device__ __forceinline__ int pair_pages(const Params &p, int n, int k) {
     const int pages = (p.eff_len[n] + p.block_size - 1) / p.block_size - prefix_pages_of(p, n);
@@ -356,8 +368,8 @@ struct LdsVec<8> { typedef u32x2 T; };
 template <>
 struct LdsVec<4> { typedef uint32_t T; };
 
-// Persistent split-K decode for bf16 / fp8 pools, D in {64, 128}, block_size 16,
-// G = H/Hkv in {1, 2, 4, 8}.  The grid holds a fixed number of one-wave
+// Persistent split-K decode for bf16 / fp8 / f32 pools, D in {64, 128},
+// block_size 16, G = H/Hkv in {1, 2, 4, 8}.  The grid holds a fixed number of one-wave
 // workgroups; each loops over work items.  Per item, the partition's pages
 // stream through kStages LDS stages per wave: every page (K and V, 16 rows of
 // D elements each) arrives by global_load_lds_dwordx4, 1 KiB contiguous per
@@ -385,12 +397,26 @@ struct LdsVec<4> { typedef uint32_t T; };
 //         DT*m + dt.
 // fp8 pools: the K scale folds into the softmax scale, the V scale into the
 // result.
-template <int KV, int D, int G>
+// f32 pools: QK^T and PV on v_mfma_f32_16x16x4_f32, four k-steps per 16-byte
+// chunk, with V's dims of a lane chosen so that its LDS reads are contiguous
+// over 16 lanes; the scores' fragment is P^T's, as above.  64 MFMAs of 32 cycles
+// a page are 0.85 us, hidden behind the 2.3 us that a page takes at the HBM rate
+// with one wave a SIMD.  48 x 128..4096 tokens, 32 / 8 heads of 128: 2500 us in
+// decode_generic_kernel (a row per lane: uncoalesced, serial), 158 us here
+// (5.5 TB/s).
+// DIRECT: no plan and no queue; workgroup (kvh, part, n) is partition `part` of
+// sequence n (at most kDirectPages pages), derives its pages from the length
+// and the table itself and ends.  A partition whose pages end at an invalid
+// table entry marks its partial (sign bit of l), and the reduce drops the
+// partitions after it.
+template <int KV, int D, int G, bool DIRECT>
 __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     constexpr int BS = 16;
-    constexpr int ELT = KV == ZK_BF16 ? 2 : 1;
+    constexpr int BIDS = DIRECT ? kDirectPages : kMaxItemPages;
+    constexpr bool F32 = KV == ZK_F32;
+    constexpr int ELT = F32 ? 4 : KV == ZK_BF16 ? 2 : 1;
     constexpr int DG = D / 4;            // head dims per lane group in QK
-    constexpr int KK = DG / 8;           // MFMA k-steps
+    constexpr int KK = F32 ? D / 16 : DG / 8;  // 16-byte Q chunks per lane (bf16: MFMA k-steps)
     constexpr int DT = D / 16;           // PV dim tiles = dims per lane per V row
     constexpr int RB = D * ELT;          // bytes per token row
     constexpr int CPR = RB / 16;         // 16-byte chunks per row
@@ -401,10 +427,13 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     constexpr int KCH = KBYTES / 16;     // ... in 16-byte chunks
     constexpr int VTB = DT * ELT;        // V bytes per lane per token row
     static_assert(PAGE % 1024 == 0 && KBYTES % 16 == 0 && DT % 2 == 0, "page shape");
-    typedef typename LdsVec<VTB>::T vtrow_t;
+    typedef typename LdsVec<F32 ? 16 : VTB>::T vtrow_t;
+    constexpr int VR = F32 ? VTB / 16 : 1;  // V reads per lane and token row
     typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef typename std::conditional<F32, f32x4, bf16x8>::type qfrag_t;  // 16 bytes of a query row
+    const qfrag_t qzero = __builtin_bit_cast(qfrag_t, u32x4{0u, 0u, 0u, 0u});
     __shared__ __attribute__((aligned(16))) char lds[kStages][2][PAGE];  // [stage][K|V]
-    __shared__ int32_t bids[kMaxItemPages];                              // this item's block ids
+    __shared__ int32_t bids[BIDS];                              // this item's block ids
 
     const int lane = threadIdx.x, col = lane & 15, grp = lane >> 4;
     const int H = p.num_heads, Hkv = p.num_kv_heads;
@@ -420,10 +449,14 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     uint32_t kl[KCH];  // LDS offsets of this lane's K fragment chunks
 #pragma unroll
     for (int f = 0; f < KCH; ++f) {
-        const int row = col, c = grp * KCH + f;
+        // bf16 / fp8: lane group grp holds dims DG grp .. of the row; f32: dims
+        // 16 f + 4 grp .. of chunk f, so consecutive chunks feed consecutive k-steps
+        const int row = col, c = F32 ? 4 * f + grp : grp * KCH + f;
         kl[f] = (row * CPR + (c ^ (row % CPR))) * 16;
     }
-    const uint32_t vt_off = (uint32_t)((4 * grp) * RB + col * VTB);  // + i * RB
+    // + i * RB; f32: + 256 h, dims 64 h + 4 col .. + 3 (16 lanes read one
+    // contiguous 256-byte piece)
+    const uint32_t vt_off = (uint32_t)((4 * grp) * RB + col * (F32 ? 16 : VTB));
 
     // Wait until page pi of an np-page item has landed in LDS: the pages
     // issued after it (up to kStages - 1) may still be in flight.
@@ -444,11 +477,11 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     // holding a long item reserve a short one it only starts much later,
     // while waves that finish their short items find the queue empty: with
     // mixed item lengths that left a tail of late short items.)
-    const int nq = p.queues, xq = blockIdx.x % nq;
+    const int nq = DIRECT ? 1 : p.queues, xq = blockIdx.x % nq;
     auto head = [&](int q) { return p.work + kQueueStride * (1 + q + p.head_set * kQueues); };
     // the other set of heads back to its start for the next launch on this
     // workspace (no wave of this launch touches it)
-    if (blockIdx.x == 0 && lane < nq)
+    if (!DIRECT && blockIdx.x == 0 && lane < nq)
         p.work[kQueueStride * (1 + lane + (1 - p.head_set) * kQueues)] = (p.num_waves - lane + nq - 1) / nq;
     auto claim_next = [&]() {
         if (lane == 0) next = atomicAdd(head(xq), 1);
@@ -493,7 +526,20 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     };
 
     // B fragment of query row (n, qh): this lane group's DG dims as KK bf16x8.
-    auto load_q = [&](size_t qr, int qh, bf16x8 *qf) {
+    auto load_q = [&](size_t qr, int qh, qfrag_t *qf) {
+        if constexpr (F32) {
+            const size_t qb = qr * (size_t)p.q_stride + (size_t)qh * D + 4 * grp;
+#pragma unroll
+            for (int j = 0; j < KK; ++j) {
+                if (p.q_f32) {
+                    qf[j] = *reinterpret_cast<const f32x4 *>((const float *)p.q + qb + 16 * j);
+                } else {
+                    const u32x2 w = *reinterpret_cast<const u32x2 *>((const uint16_t *)p.q + qb + 16 * j);
+                    qf[j] = f32x4{bf16lo(w[0]), bf16hi(w[0]), bf16lo(w[1]), bf16hi(w[1])};
+                }
+            }
+            return;
+        } else {
         const size_t qb = qr * (size_t)p.q_stride + (size_t)qh * D + (size_t)grp * DG;
         if (p.q_f32) {
             const float *qq = (const float *)p.q + qb;
@@ -509,9 +555,10 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8 *>(qq + 8 * kk);
         }
+        }
     };
 
-    const int total = *(cint_t)p.work;
+    const int total = DIRECT ? 0 : *(cint_t)p.work;
     // The next item and its descriptor, loaded while the current item's last
     // page is computed (the claim has returned by then).  The scalar load is
     // issued by inline asm: a plain load, whose result is only used after the
@@ -564,7 +611,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     // registers (lane c < CPR: chunk c of K, CPR <= lane < 2 CPR: of V); it is
     // written into the page's LDS copy once that has landed, and to the pools
     // at byte offset row_dst of the K / V pool.
-    auto attend = [&]<int T>(const bf16x8 (&qf)[T][KK], const int32_t *trow, int4 blk0, int page0, int np, int len,
+    auto attend = [&]<int T>(const qfrag_t (&qf)[T][KK], const int32_t *trow, int4 blk0, int page0, int np, int len,
                              int kvh, float sl2, f32x4 (&o)[DT][T], float (&m)[T], float (&l)[T], int fuse_tib,
                              u32x4 nrow, size_t row_dst) {
         const char *kbase = p.k_pool + ((size_t)kvh * PAGE);
@@ -606,10 +653,14 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) kw[4 * f + j] = c4[j];
             }
-            vtrow_t vt[4];  // token rows 4*grp+i, dims DT*col .. DT*col+DT-1
+            // token rows 4*grp+i, dims DT*col .. DT*col+DT-1 (f32: see vt_off)
+            vtrow_t vt[4][VR];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) vt[i] = *reinterpret_cast<const vtrow_t *>(lds[s][1] + vt_off + i * RB);
-            const int nb = bids[min(pi + kStages, kMaxItemPages - 1)];
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int h = 0; h < VR; ++h)
+                    vt[i][h] = *reinterpret_cast<const vtrow_t *>(lds[s][1] + vt_off + i * RB + 256 * h);
+            const int nb = bids[min(pi + kStages, BIDS - 1)];
             // The stage is free once its reads are done: the empty asm needs
             // their results, so the compiler's own lgkmcnt wait lands here
             // (it does not count an explicit s_waitcnt as completing them and
@@ -617,15 +668,37 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
             for (int j = 0; j < KBYTES / 4; ++j) asm volatile("" ::"v"(kw[j]));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(vt[i]));
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int h = 0; h < VR; ++h) asm volatile("" ::"v"(vt[i][h]));
             asm volatile("" ::"v"(nb));
             if (pi + kStages < np) issue_blk(__builtin_amdgcn_readfirstlane(nb), s);
-            if (pi == np - 1 - kStages) claim_next();
-            if (pi == np - 1) fetch_next();
+            if constexpr (!DIRECT) {
+                if (pi == np - 1 - kStages) claim_next();
+                if (pi == np - 1) fetch_next();
+            }
 
             f32x4 sacc[T];
 #pragma unroll
             for (int t = 0; t < T; ++t) sacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (F32) {
+                // k-step (f, e): lane group grp holds dim 16 f + 4 grp + e of
+                // its K row (A) and query row (B); two chains a tile
+                f32x4 s2[T];
+#pragma unroll
+                for (int t = 0; t < T; ++t) s2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int f = 0; f < KCH; ++f)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int t = 0; t < T; ++t) {
+                            f32x4 &a = e & 1 ? s2[t] : sacc[t];
+                            a = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(kw[4 * f + e]), qf[t][f][e], a, 0, 0, 0);
+                        }
+#pragma unroll
+                for (int t = 0; t < T; ++t) sacc[t] += s2[t];
+            } else {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
                 u32x4 w;
@@ -640,12 +713,15 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                     sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), qf[t][kk],
                                                                       sacc[t], 0, 0, 0);
             }
-            // V rows as bf16 pairs: w[i][j] = dims (2j, 2j+1) of token row 4*grp+i
-            uint32_t w[4][DT / 2];
+            }
+            // V rows as bf16 pairs: w[i][j] = dims (2j, 2j+1) of token row
+            // 4*grp+i; f32: the DT values themselves
+            constexpr int VW = F32 ? DT : DT / 2;
+            uint32_t w[4][VW];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if constexpr (KV == ZK_BF16) {
-                    __builtin_memcpy(w[i], &vt[i], 2 * DT);
+                if constexpr (KV != ZK_FP8_E4M3) {
+                    __builtin_memcpy(w[i], &vt[i], 4 * VW);
                 } else {
                     uint32_t b8[DT / 4];
                     __builtin_memcpy(b8, &vt[i], DT);
@@ -663,9 +739,10 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 for (int i = 0; i < 4; ++i)
                     if (tok0 + i >= len)
 #pragma unroll
-                        for (int j = 0; j < DT / 2; ++j) w[i][j] = 0u;
+                        for (int j = 0; j < VW; ++j) w[i][j] = 0u;
             }
-            s16x4 va[DT];  // element i of tile dt = V[4*grp+i][DT*col+dt]
+            s16x4 va[F32 ? 1 : DT];  // element i of tile dt = V[4*grp+i][DT*col+dt]
+            if constexpr (!F32)
 #pragma unroll
             for (int j = 0; j < DT / 2; ++j) {
                 const u32x2 lo{__builtin_amdgcn_perm(w[1][j], w[0][j], 0x05040100u),
@@ -697,10 +774,19 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) pr[i] = exp2_fast(sc[i] - m[t]);
                 l[t] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+                if constexpr (F32) {
+                    // k-step i: V^T column token 4*grp+i (A) and its weight (B)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int dt = 0; dt < DT; ++dt)
+                            o[dt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w[i][dt]), pr[i], o[dt][t], 0, 0, 0);
+                    continue;
+                }
                 const s16x4 pb = __builtin_bit_cast(s16x4, u32x2{bf16x2_rne(pr[0], pr[1]), bf16x2_rne(pr[2], pr[3])});
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
-                    o[dt][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[dt], pb, o[dt][t], 0, 0, 0);
+                    o[dt][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[F32 ? 0 : dt], pb, o[dt][t], 0, 0, 0);
             }
         };
         // the first pages straight from the descriptor, then the other ids
@@ -709,7 +795,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
         for (int j = 0; j < kStages; ++j)
             if (j < np) issue_blk(b0[j], j);
-        stage_bids(trow, np);
+        if constexpr (!DIRECT) stage_bids(trow, np);  // (DIRECT: staged by the caller)
         // Q is complete before the loop on every path (see stage_bids)
 #pragma unroll
         for (int t = 0; t < T; ++t)
@@ -717,7 +803,8 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             for (int kk = 0; kk < KK; ++kk) asm volatile("" ::"v"(qf[t][kk]));
         // and so is the fused row
         asm volatile("" ::"v"(nrow[0]), "v"(nrow[1]), "v"(nrow[2]), "v"(nrow[3]));
-        if (np <= kStages) claim_next();
+        if constexpr (!DIRECT)
+            if (np <= kStages) claim_next();
         // one page per iteration (a single loop-carried accumulator set)
         for (int pi = 0, st = 0; pi < np; ++pi, st = (st + 1 == kStages ? 0 : st + 1)) page(pi, st);
 #pragma unroll
@@ -728,8 +815,19 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     };
 
     // Lane (grp, col) holds dims DT*(4*grp+i)+dt, i < 4, dt < DT, of row col:
-    // four runs of DT consecutive floats.
+    // four runs of DT consecutive floats.  f32 pools: tile dt = 4 h + e is dims
+    // 64 h + 4*(4*grp+i) + e, runs of four.
     auto store_row_f32 = [&](float *dst, const f32x4 (&o)[DT][2], int t, float scale) {
+        if constexpr (F32) {
+#pragma unroll
+            for (int h = 0; h < DT / 4; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const f32x4 v = f32x4{o[4 * h][t][i], o[4 * h + 1][t][i], o[4 * h + 2][t][i], o[4 * h + 3][t][i]} * scale;
+                    __builtin_memcpy(dst + 64 * h + 16 * grp + 4 * i, &v, sizeof(v));
+                }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float v[DT];
@@ -745,13 +843,106 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     };
     const u32x4 no_row = {0u, 0u, 0u, 0u};
 
+    // a sequence's own partition: rows 0..G-1 are its heads of kv-head kvh
+    // (ns shared and nparts own partitions in all; cut: the partition's pages
+    // end at an invalid table entry)
+    auto own_part = [&](int n, int kvh, int part, int page0, int np, int len, int ns, int nparts, int4 d1, bool cut) {
+        const int qh = qhead_of(p, kvh, col % G, G);
+        const size_t qr = q_row(n);
+        qfrag_t qf[1][KK];
+        if (col < G) load_q(qr, qh, qf[0]);
+        else
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) qf[0][kk] = qzero;
+        float sl2 = p.scale_log2, vscale = 1.0f;
+        if constexpr (KV == ZK_FP8_E4M3) {
+            sl2 *= ((cfloat_t)p.k_scales)[(size_t)n * Hkv + kvh];
+            vscale = ((cfloat_t)p.v_scales)[(size_t)n * Hkv + kvh];
+        }
+        // fused append: the item holding the sequence's last page
+        int fuse_tib = -1;
+        u32x4 nrow = no_row;
+        size_t row_dst = 0;
+        if constexpr (KV == ZK_BF16) {
+            if (p.new_k && len > 0 && np > 0 && page0 + np == (len + BS - 1) / BS) {
+                fuse_tib = (len - 1) % BS;
+                const int blk = ((cint_t)p.bt)[(size_t)n * p.max_blocks + (len - 1) / BS];
+                const int c = lane % CPR;
+                row_dst = ((size_t)blk * Hkv + kvh) * PAGE + (size_t)fuse_tib * RB + (size_t)c * 16;
+                if (lane < 2 * CPR)
+                    nrow = *reinterpret_cast<const u32x4 *>((lane < CPR ? p.new_k : p.new_v) +
+                                                            (size_t)n * p.new_row_bytes + (size_t)kvh * RB + c * 16);
+            }
+        }
+        f32x4 o[DT][1];
+        float m[1], l[1];
+        attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, kvh, sl2,
+                                      o, m, l, fuse_tib, nrow, row_dst);
+        if (col < G) {
+            if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
+                const float inv = l[0] > 0.0f ? vscale / l[0] : 0.0f;
+                const size_t ob = (qr * H + qh) * D;
+                if (p.q_f32) {
+                    f32x4 o2[DT][2];
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) o2[dt][0] = o[dt][0];
+                    store_row_f32((float *)p.out + ob, o2, 0, inv);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        uint32_t v[DT / 2];
+#pragma unroll
+                        for (int j = 0; j < DT / 2; ++j)
+                            v[j] = bf16x2_rne(o[2 * j][0][i] * inv, o[2 * j + 1][0][i] * inv);
+                        if constexpr (F32) {
+#pragma unroll
+                            for (int h = 0; h < DT / 4; ++h)
+                                __builtin_memcpy((uint16_t *)p.out + ob + 64 * h + 16 * grp + 4 * i, v + 2 * h, 8);
+                        } else {
+                            __builtin_memcpy((uint16_t *)p.out + ob + DT * (4 * grp + i), v, sizeof(v));
+                        }
+                    }
+                }
+            } else {
+                const size_t slot = ((size_t)n * H + qh) * p.max_parts + ns + part;
+                f32x4 o2[DT][2];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) o2[dt][0] = o[dt][0];
+                store_partial(slot, o2, 0, vscale, m[0], cut ? -l[0] : l[0]);
+            }
+        }
+    };
+
+    if constexpr (DIRECT) {
+        const int kvh = blockIdx.x, part = blockIdx.y, n = blockIdx.z;
+        const int page0 = part * p.part_pages;
+        const int32_t *row = p.bt + (size_t)n * p.max_blocks;
+        // this lane's page id beside the length: one round trip
+        const int e = page0 + lane < p.max_blocks ? row[page0 + lane] : -1;
+        const int len = min(max(((cint_t)p.seq_lens)[n], 0), p.max_blocks * BS);
+        const int pages = (len + BS - 1) / BS, nparts = (pages + p.part_pages - 1) / p.part_pages;
+        if (part >= max(1, nparts)) return;
+        const int want = min(p.part_pages, pages - page0);
+        const uint64_t bad = __builtin_amdgcn_ballot_w64(lane < want && (e < 0 || (int64_t)e >= p.num_blocks));
+        const int np = bad ? min(want, (int)__builtin_ctzll(bad)) : want;
+        bids[lane] = e;
+        static_assert(kDirectPages == kWave, "one table entry per lane");
+        wait_lgkmcnt0();  // visible to this wave's own reads
+        const int4 first = make_int4(__builtin_amdgcn_readlane(e, 0), __builtin_amdgcn_readlane(e, 1),
+                                     __builtin_amdgcn_readlane(e, 2), __builtin_amdgcn_readlane(e, 3));
+        own_part(n, kvh, part, page0, np, len, 0, nparts, first, bad != 0);
+        return;
+    }
+
     int item = blockIdx.x;  // first item static, the rest from the queue
     int4 d0 = make_int4(0, 0, 0, 0), d1 = make_int4(0, 0, 0, 0);
     if (item < total) load_desc(item / Hkv, d0, d1);
     while (item < total) {
         const int kvh = item % Hkv;
         have_next = false;
-        if (KV == ZK_BF16 && d0.x < 0) {
+        bool own = true;
+        if constexpr (KV == ZK_BF16) own = d0.x >= 0;
+        if (!own) {
             // shared-prefix partition of subgroup sg: up to 32 rows, member-major
             const int sg = -1 - d0.x, part = d0.y, n0 = d0.z, np = d0.w;
             const int page0 = part * p.shared_part_pages;
@@ -762,7 +953,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             int mem_s[NM];
 #pragma unroll
             for (int j = 0; j < NM; ++j) mem_s[j] = cmem[j];
-            bf16x8 qf[2][KK];
+            qfrag_t qf[2][KK];
             int nm[2];  // member of this lane's row in tile t, or -1
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -774,7 +965,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 if (nm[t] >= 0) load_q(q_row(nm[t]), qhead_of(p, kvh, r % G, G), qf[t]);
                 else
 #pragma unroll
-                    for (int kk = 0; kk < KK; ++kk) qf[t][kk] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+                    for (int kk = 0; kk < KK; ++kk) qf[t][kk] = qzero;
             }
             f32x4 o[DT][2];
             float m[2], l[2];
@@ -789,71 +980,13 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 }
             }
         } else {
-            // a sequence's own partition: rows 0..G-1 are its heads of kv-head kvh
             const int n = d0.x, part = d0.y, page0 = d0.z, np = d0.w;
             const int len = ((cint_t)p.eff_len)[n];  // walk already cut at the first invalid entry
             const int pb = p.seq_pb ? ((cint_t)p.seq_pb)[n] : 0;
             const int ns = pb > 0 ? (pb + p.shared_part_pages - 1) / p.shared_part_pages : 0;
             const int rest = (len + p.block_size - 1) / p.block_size - pb;
             const int nparts = rest > 0 ? (rest + p.part_pages - 1) / p.part_pages : 0;
-            const int qh = qhead_of(p, kvh, col % G, G);
-            const size_t qr = q_row(n);
-            bf16x8 qf[1][KK];
-            if (col < G) load_q(qr, qh, qf[0]);
-            else
-#pragma unroll
-                for (int kk = 0; kk < KK; ++kk) qf[0][kk] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-            float sl2 = p.scale_log2, vscale = 1.0f;
-            if constexpr (KV == ZK_FP8_E4M3) {
-                sl2 *= ((cfloat_t)p.k_scales)[(size_t)n * Hkv + kvh];
-                vscale = ((cfloat_t)p.v_scales)[(size_t)n * Hkv + kvh];
-            }
-            // fused append: the item holding the sequence's last page
-            int fuse_tib = -1;
-            u32x4 nrow = no_row;
-            size_t row_dst = 0;
-            if constexpr (KV == ZK_BF16) {
-                if (p.new_k && len > 0 && np > 0 && page0 + np == (len + BS - 1) / BS) {
-                    fuse_tib = (len - 1) % BS;
-                    const int blk = ((cint_t)p.bt)[(size_t)n * p.max_blocks + (len - 1) / BS];
-                    const int c = lane % CPR;
-                    row_dst = ((size_t)blk * Hkv + kvh) * PAGE + (size_t)fuse_tib * RB + (size_t)c * 16;
-                    if (lane < 2 * CPR)
-                        nrow = *reinterpret_cast<const u32x4 *>((lane < CPR ? p.new_k : p.new_v) +
-                                                                (size_t)n * p.new_row_bytes + (size_t)kvh * RB + c * 16);
-                }
-            }
-            f32x4 o[DT][1];
-            float m[1], l[1];
-            attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, kvh, sl2,
-                                          o, m, l, fuse_tib, nrow, row_dst);
-            if (col < G) {
-                if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
-                    const float inv = l[0] > 0.0f ? vscale / l[0] : 0.0f;
-                    const size_t ob = (qr * H + qh) * D;
-                    if (p.q_f32) {
-                        f32x4 o2[DT][2];
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt) o2[dt][0] = o[dt][0];
-                        store_row_f32((float *)p.out + ob, o2, 0, inv);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            uint32_t v[DT / 2];
-#pragma unroll
-                            for (int j = 0; j < DT / 2; ++j)
-                                v[j] = bf16x2_rne(o[2 * j][0][i] * inv, o[2 * j + 1][0][i] * inv);
-                            __builtin_memcpy((uint16_t *)p.out + ob + DT * (4 * grp + i), v, sizeof(v));
-                        }
-                    }
-                } else {
-                    const size_t slot = ((size_t)n * H + qh) * p.max_parts + ns + part;
-                    f32x4 o2[DT][2];
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) o2[dt][0] = o[dt][0];
-                    store_partial(slot, o2, 0, vscale, m[0], l[0]);
-                }
-            }
+            own_part(n, kvh, part, page0, np, len, ns, nparts, d1, false);
         }
         if (!have_next) fetch_next();  // an item without pages
         item = nx;
@@ -1120,14 +1253,16 @@ __global__ void __launch_bounds__(kWave) decode_reduce_vec_kernel(Params p) {
 // head's (m, l) of every partition itself (no cross-lane reductions) and the
 // first C partitions' partials with them, one memory round trip; partitions
 // are added in slot order.
-template <int D, int G>
+// MARKS: a partition marked by the sign of its l (planless launches) is the
+// context's last.
+template <int D, int G, bool MARKS>
 __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     constexpr int LPH = kWave / G, F = G * D / kWave, F4 = F / 4;
     constexpr int C = 8;  // partitions loaded with the (m, l)
     static_assert(F % 4 == 0 && kWave % G == 0, "lane layout");
     const int kvh = blockIdx.x, n = blockIdx.y, lane = threadIdx.x;
     const int ns = shared_parts_of(p, n);
-    const int nparts = ns + private_parts_of(p, n);
+    int nparts = ns + private_parts_of<MARKS>(p, n);
     if (ns == 0 && nparts <= 1) return;  // written by the partition kernel
     const int hh = lane / LPH, d0 = (lane % LPH) * F;
     const int qh = qhead_of(p, kvh, hh, G);
@@ -1145,9 +1280,25 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
         }
     }
     float M = -INFINITY;
+    if constexpr (MARKS) {
 #pragma unroll
-    for (int i = 0; i < C; ++i) M = fmaxf(M, ml[i].x);
-    for (int i = C; i < nparts; ++i) M = fmaxf(M, p.ml[base + i].x);
+        for (int i = C - 1; i >= 0; --i)
+            if (i < nparts && signbit(ml[i].y)) nparts = i + 1;
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            M = i < nparts ? fmaxf(M, ml[i].x) : M;
+            ml[i].y = fabsf(ml[i].y);
+        }
+        for (int i = C; i < nparts; ++i) {
+            const float2 v = p.ml[base + i];
+            M = fmaxf(M, v.x);
+            if (signbit(v.y)) nparts = i + 1;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < C; ++i) M = fmaxf(M, ml[i].x);
+        for (int i = C; i < nparts; ++i) M = fmaxf(M, p.ml[base + i].x);
+    }
     auto weight = [&](float2 v) { return v.x == -INFINITY ? 0.0f : exp2f(v.x - M); };
     float L = 0.0f;
     f32x4 acc[F4];
@@ -1166,7 +1317,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     for (int i = C; i < nparts; ++i) {
         const float2 v = p.ml[base + i];
         const float w = weight(v);
-        L += v.y * w;
+        L += (MARKS ? fabsf(v.y) : v.y) * w;
 #pragma unroll
         for (int k = 0; k < F4; ++k) {
             const f32x4 y = *reinterpret_cast<const f32x4 *>(p.po + (base + i) * D + d0 + 4 * k);
@@ -1191,6 +1342,70 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
         }
         __builtin_memcpy((uint16_t *)p.out + ob, v, sizeof(v));
     }
+}
+
+// The merge for sequences of many partitions (long contexts in small batches):
+// one 256-thread workgroup per (q-head, sequence), LP = D / 4 lanes a
+// partition, so 256 / LP partitions a load and U loads in flight per thread;
+// each wave reads all (m, l) itself, and the groups' sums meet in LDS.
+template <int D>
+__global__ void __launch_bounds__(256) decode_reduce_many_kernel(Params p) {
+    constexpr int LP = D / 4, PG = 256 / LP, U = 8;
+    __shared__ f32x4 part_sum[256];
+    const int h = blockIdx.x, n = blockIdx.y, t = threadIdx.x, lane = t & 63;
+    const int ns = shared_parts_of(p, n);
+    int nparts = ns + (p.eff_len ? private_parts_of(p, n) : private_parts_of<true>(p, n));
+    if (ns == 0 && nparts <= 1) return;  // written by the partition kernel
+    const size_t base = ((size_t)n * p.num_heads + h) * p.max_parts;
+    const int g = t / LP, d0 = 4 * (t % LP);
+    auto load = [&](int i) { return *reinterpret_cast<const f32x4 *>(p.po + (base + i) * D + d0); };
+    f32x4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = load(min(u * PG + g, nparts - 1));  // beside the (m, l)
+    // the first marked partition (sign of l) ends the context
+    int last = nparts - 1;
+    for (int i = lane; i < nparts; i += kWave)
+        if (signbit(p.ml[base + i].y)) last = min(last, i);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) last = min(last, __shfl_xor(last, o));
+    nparts = last + 1;
+    float M = -INFINITY;
+    for (int i = lane; i < nparts; i += kWave) M = fmaxf(M, p.ml[base + i].x);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+    auto weight = [&](float m) { return m == -INFINITY ? 0.0f : exp2f(m - M); };
+    float L = 0.0f;
+    for (int i = lane; i < nparts; i += kWave) {
+        const float2 v = p.ml[base + i];
+        L += fabsf(v.y) * weight(v.x);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < nparts; i0 += PG * U) {
+        float w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * PG + g;
+            if (i0 > 0) x[u] = load(min(i, nparts - 1));
+            w[u] = weight(p.ml[base + min(i, nparts - 1)].x);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * PG + g < nparts)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[c] = fmaf(w[u], x[u][c], acc[c]);
+    }
+    part_sum[t] = acc;
+    __syncthreads();
+    if (t >= LP) return;
+    acc = part_sum[t];
+#pragma unroll
+    for (int q = 1; q < PG; ++q) acc += part_sum[q * LP + t];
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const size_t ob = (qrow(p, n) * p.num_heads + h) * D + d0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) store_out(p, ob + c, acc[c] * inv);
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1254,25 +1469,38 @@ int persistent_grid() {
     return cus * 4 * waves_per_simd_config();
 }
 
+template <int KV, int D, int G>
+void launch_mfma_k(const Params &p, hipStream_t s) {
+    if (p.num_waves > 0)
+        decode_mfma_kernel<KV, D, G, false><<<p.num_waves, kWave, 0, s>>>(p);
+    else
+        decode_mfma_kernel<KV, D, G, true><<<dim3(p.num_kv_heads, p.max_parts, p.num_seqs), kWave, 0, s>>>(p);
+}
+
 template <int KV, int D>
-bool launch_mfma_g(const Params &p, int grid, hipStream_t s, int G) {
+void launch_mfma_g(const Params &p, hipStream_t s, int G) {
     switch (G) {
-        case 1: decode_mfma_kernel<KV, D, 1><<<grid, kWave, 0, s>>>(p); return true;
-        case 2: decode_mfma_kernel<KV, D, 2><<<grid, kWave, 0, s>>>(p); return true;
-        case 4: decode_mfma_kernel<KV, D, 4><<<grid, kWave, 0, s>>>(p); return true;
-        case 8: decode_mfma_kernel<KV, D, 8><<<grid, kWave, 0, s>>>(p); return true;
-        default: return false;
+        case 1: launch_mfma_k<KV, D, 1>(p, s); break;
+        case 2: launch_mfma_k<KV, D, 2>(p, s); break;
+        case 4: launch_mfma_k<KV, D, 4>(p, s); break;
+        default: launch_mfma_k<KV, D, 8>(p, s); break;
     }
 }
 
 template <int KV>
-bool launch_mfma(const Params &p, int grid, hipStream_t s, int G) {
-    if (p.head_dim == 128) return launch_mfma_g<KV, 128>(p, grid, s, G);
-    return launch_mfma_g<KV, 64>(p, grid, s, G);
+void launch_mfma(const Params &p, hipStream_t s, int G) {
+    if (p.head_dim == 128) launch_mfma_g<KV, 128>(p, s, G);
+    else launch_mfma_g<KV, 64>(p, s, G);
+}
+
+template <int G>
+void launch_reduce_kv(const Params &p, dim3 grid, hipStream_t s) {
+    if (p.eff_len) decode_reduce_kv_kernel<128, G, false><<<grid, kWave, 0, s>>>(p);
+    else decode_reduce_kv_kernel<128, G, true><<<grid, kWave, 0, s>>>(p);
 }
 
 bool mfma_supported(int kv_dtype, int head_dim, int block_size, int G) {
-    return (kv_dtype == ZK_BF16 || kv_dtype == ZK_FP8_E4M3) && block_size == 16 &&
+    return valid_dtype(kv_dtype) && block_size == 16 &&
            (head_dim == 128 || head_dim == 64) && (G == 1 || G == 2 || G == 4 || G == 8);
 }
 
@@ -1282,6 +1510,37 @@ int check_launch(const char *what) {
         return set_error(ZK_ERR_HIP, std::string("Internal error: ") + what + ": " + hipGetErrorString(e));
     return ZK_OK;
 }
+
+// Planless launches: partitions of a sequence for `units` (capacity) pages
+// over all sequences and kv-heads, of page_bytes of K and V each; 0: too much
+// work for one.  The host knows the tables' capacity, not the lengths.
+//
+// Against the planned persistent grid a planless launch saves the table walk
+// and plan kernels (7-50 us) and hides an item's prologue behind other
+// resident waves, but starts items in table order, not longest first.
+// Measured (planned / planless, us): 2 x 26000 bf16 tokens 94 / 38, 4 x 17..1000
+// 22 / 15, 64 x 512..8192 bf16 177 / 165, fp8 116 / 89, f32 324 / 313; 40 x
+// 1024..16384 206 / 193; then 192 x 300..4000 bf16 264 / 278 and 256 x 512..8192
+// 643 / 708: the line lies at 3 GB of capacity.
+//
+// The partition length P balances the items' fixed cost, (units / P) a / waves,
+// against the tail of one item, P b: P ~ sqrt(units), with page_bytes for the
+// page time.  sqrt(bytes) / 1000 is within 5 % of the best of 4, 8, 16, 24, 32,
+// 48, 64 on bf16, fp8 and f32, 128 and 64 dims, 8000 to 260000 pages.  Fewer
+// than 8 pages do not pay for the reduce; the count is rounded to the nearest
+// so that a table a little over P stays one partition (no reduce at all).
+constexpr double kDirectBytes = 3e9;
+int direct_parts(double units, double page_bytes, int max_blocks) {
+    const double bytes = units * page_bytes;
+    if (bytes > kDirectBytes) return 0;
+    const double pp = std::min((double)kDirectPages, std::max(8.0, std::sqrt(bytes) * 1e-3));
+    return std::max((max_blocks + kDirectPages - 1) / kDirectPages, std::max(1, (int)(max_blocks / pp + 0.5)));
+}
+
+// Partitions from which one workgroup a q-head merges them: eight lines of a
+// wave's loads in flight instead of a serial walk (2 sequences of 125
+// partitions: 35 -> 5 us).
+constexpr int kManyParts = 16;
 
 // Pages per shared-prefix item: about one item per two waves over all
 // subgroups' pages, so half the waves stream the shared pages (two query-row
@@ -1305,9 +1564,13 @@ int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves)
 size_t zk::paged_decode_workspace(int num_seqs, int num_heads, int head_dim, int max_blocks_per_seq,
                                   int block_size, bool shared) {
     if (num_seqs <= 0 || num_heads <= 0 || head_dim <= 0 || max_blocks_per_seq <= 0) return 256;
-    return ws_layout(num_seqs, num_heads, head_dim,
-                     max_parts_for(max_blocks_per_seq, min_part_pages(head_dim, block_size)) + (shared ? 1 : 0))
-        .total;
+    // the planned paths' partitions, or (16-token blocks of 64 or 128 dims) the
+    // planless one's at the fewest bytes a page and the most heads a kv-head
+    int parts = max_parts_for(max_blocks_per_seq, min_part_pages(head_dim, block_size)) + (shared ? 1 : 0);
+    if (block_size == 16 && (head_dim == 64 || head_dim == 128))
+        parts = std::max(parts, direct_parts((double)num_seqs * max_blocks_per_seq * std::max(1, num_heads / 8),
+                                             2.0 * block_size * head_dim, max_blocks_per_seq));
+    return ws_layout(num_seqs, num_heads, head_dim, parts).total;
 }
 
 bool zk::paged_decode_shares_prefixes(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads) {
@@ -1348,17 +1611,20 @@ int check_decode_args(zk_dtype q_dtype, zk_dtype kv_dtype, int num_seqs, int num
 // Which kernel a call runs, how it cuts the contexts and the workspace it
 // needs (arguments already checked).
 struct DecodeShape {
-    bool use_mfma, shared;
+    bool use_mfma, shared, direct;
     int part_pages, shared_pages, max_parts, waves;
     WsLayout w;
 };
 // max_waves > 0 caps the MFMA path's persistent grid (partitions are sized
 // for the waves that run them).
 DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num_kv_heads, int head_dim,
-                         int block_size, int max_blocks_per_seq, const PrefixGroups *pg, int max_waves = 0) {
+                         int block_size, int max_blocks_per_seq, const PrefixGroups *pg, bool aligned,
+                         size_t workspace_bytes, int max_waves = 0) {
     DecodeShape d;
     const int G = num_heads / num_kv_heads;
-    d.use_mfma = mfma_supported(kv_dtype, head_dim, block_size, G);
+    // f32 pools: any alignment was and is accepted, the 16-byte accesses of
+    // the MFMA kernel need theirs
+    d.use_mfma = mfma_supported(kv_dtype, head_dim, block_size, G) && (kv_dtype != ZK_F32 || aligned);
     d.waves = persistent_grid();
     if (max_waves > 0 && max_waves < d.waves) d.waves = max_waves;
     d.part_pages = d.use_mfma ? mfma_part_pages(num_seqs, num_kv_heads, max_blocks_per_seq, d.waves)
@@ -1370,6 +1636,19 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
     d.max_parts = d.shared ? max_parts_for(max_blocks_per_seq, min_part_pages(head_dim, block_size)) + 1
                            : max_parts_for(max_blocks_per_seq, d.part_pages);
     d.w = ws_layout(num_seqs, num_heads, head_dim, d.max_parts);
+    d.direct = false;
+    if (d.use_mfma && !d.shared && max_waves == 0 && !part_pages_env()) {
+        const int parts = direct_parts((double)num_seqs * max_blocks_per_seq * num_kv_heads,
+                                       2.0 * block_size * head_dim * elt_size(kv_dtype), max_blocks_per_seq);
+        const WsLayout w = ws_layout(num_seqs, num_heads, head_dim, parts);
+        if (parts > 0 && num_seqs <= 65535 && w.total <= workspace_bytes) {
+            d.direct = true;
+            d.waves = 0;
+            d.part_pages = (max_blocks_per_seq + parts - 1) / parts;
+            d.max_parts = parts;
+            d.w = w;
+        }
+    }
     return d;
 }
 
@@ -1396,8 +1675,10 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
     if (pg && pg->num_sg > 0 && (!pg->seq_pb || !pg->sg_members || !pg->sg_pages) &&
         paged_decode_shares_prefixes(kv_dtype, head_dim, block_size, num_heads, num_kv_heads))
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged decode: NULL prefix-group array");
+    const bool aligned = (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool | (uintptr_t)out) & 15u) == 0 &&
+                         q_stride % 4 == 0;
     const DecodeShape ds = decode_shape(kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size,
-                                        max_blocks_per_seq, pg, max_waves);
+                                        max_blocks_per_seq, pg, aligned, workspace_bytes, max_waves);
     const bool use_mfma = ds.use_mfma, shared = ds.shared;
     if (append && (!use_mfma || kv_dtype != ZK_BF16 || !trusted_tables || !append->k || !append->v ||
                    append->row_bytes < (int64_t)num_kv_heads * head_dim * 2 || (append->row_bytes & 15) ||
@@ -1425,7 +1706,7 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
     p.q_stride = q_stride > 0 ? q_stride : (int64_t)num_heads * head_dim;
     p.trusted = trusted_tables ? 1 : 0;
     char *ws = (char *)workspace;
-    p.eff_len = (int32_t *)(ws + w.eff);
+    p.eff_len = ds.direct ? nullptr : (int32_t *)(ws + w.eff);
     p.items = (int4 *)(ws + w.map);
     p.work = (int32_t *)(ws + w.work);
     p.num_waves = use_mfma ? ds.waves : 0;
@@ -1457,7 +1738,7 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
 
     hipStream_t s = (hipStream_t)stream;
     reuse_plan = reuse_plan && use_mfma;
-    if (!(use_mfma && (trusted_tables || reuse_plan))) {  // trusted MFMA launches: the plan sets the lengths
+    if (!ds.direct && !(use_mfma && (trusted_tables || reuse_plan))) {  // trusted MFMA launches: the plan sets the lengths
         {
             KernelTimer timer("decode_seq_info", s);
             seq_info_kernel<<<num_seqs, kWave, 0, s>>>(p);
@@ -1465,7 +1746,12 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
         if (int rc = check_launch("zk_paged_decode seq_info")) return rc;
     }
     const bool reduce = max_parts > 1 || shared;
-    if (use_mfma) {
+    if (ds.direct) {
+        KernelTimer timer("decode_partials", s);
+        if (kv_dtype == ZK_F32) launch_mfma<ZK_F32>(p, s, G);
+        else if (kv_dtype == ZK_BF16) launch_mfma<ZK_BF16>(p, s, G);
+        else launch_mfma<ZK_FP8_E4M3>(p, s, G);
+    } else if (use_mfma) {
         // a launch reusing the plan claims from the head set the launch
         // before it put back
         reuse_plan = reuse_plan && head_set;
@@ -1479,9 +1765,9 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
         }
         {
             KernelTimer timer("decode_partials", s);
-            const int grid = p.num_waves;
-            if (kv_dtype == ZK_BF16) launch_mfma<ZK_BF16>(p, grid, s, G);
-            else launch_mfma<ZK_FP8_E4M3>(p, grid, s, G);
+            if (kv_dtype == ZK_F32) launch_mfma<ZK_F32>(p, s, G);
+            else if (kv_dtype == ZK_BF16) launch_mfma<ZK_BF16>(p, s, G);
+            else launch_mfma<ZK_FP8_E4M3>(p, s, G);
         }
         if (int rc = check_launch("zk_paged_decode partials")) return rc;
         if (head_set) *head_set = p.head_set ^ 1;
@@ -1497,9 +1783,13 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
         dim3 rgrid(num_heads, num_seqs);
         KernelTimer timer("decode_reduce", s);
         const dim3 kgrid(num_kv_heads, num_seqs);
-        if (head_dim == 128 && G == 4) decode_reduce_kv_kernel<128, 4><<<kgrid, kWave, 0, s>>>(p);
-        else if (head_dim == 128 && G == 8) decode_reduce_kv_kernel<128, 8><<<kgrid, kWave, 0, s>>>(p);
-        else if (head_dim == 128 && G == 2) decode_reduce_kv_kernel<128, 2><<<kgrid, kWave, 0, s>>>(p);
+        const bool kv_reduce = head_dim == 128 && (G == 2 || G == 4 || G == 8);
+        if (use_mfma && ((ds.direct && !kv_reduce) || max_parts > kManyParts)) {
+            if (head_dim == 128) decode_reduce_many_kernel<128><<<rgrid, 256, 0, s>>>(p);
+            else decode_reduce_many_kernel<64><<<rgrid, 256, 0, s>>>(p);
+        } else if (head_dim == 128 && G == 4) launch_reduce_kv<4>(p, kgrid, s);
+        else if (head_dim == 128 && G == 8) launch_reduce_kv<8>(p, kgrid, s);
+        else if (head_dim == 128 && G == 2) launch_reduce_kv<2>(p, kgrid, s);
         else if (head_dim == 128) decode_reduce_vec_kernel<128><<<rgrid, kWave, 0, s>>>(p);
         else if (head_dim == 64) decode_reduce_vec_kernel<64><<<rgrid, kWave, 0, s>>>(p);
         else if (head_dim == 256) decode_reduce_vec_kernel<256><<<rgrid, kWave, 0, s>>>(p);
@@ -1542,7 +1832,9 @@ int zk_paged_decode_noalloc(const void *q, zk_dtype q_dtype, const void *k_pool,
         return rc;
     if (num_seqs == 0) return ZK_OK;
     const size_t need =
-        decode_shape(kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, nullptr)
+        decode_shape(kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, nullptr,
+                     (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool | (uintptr_t)out) & 15u) == 0,
+                     (size_t)ZK_DECODE_SCRATCH_BYTES)
             .w.total;
     if (need > (size_t)ZK_DECODE_SCRATCH_BYTES)
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_paged_decode_noalloc: the call needs " +
