@@ -1462,7 +1462,9 @@ int zk_cache_attention_batch(zk_kv_cache *c, size_t layer, const char *const *id
             pre_groups = c->cus;
             dec_waves = 2 * c->cus;
         }
-        int rc = prefill_batch(c, layer, pre, pre_len, pre_off, row, q, q_dtype, q_token_stride, out, num_heads,
+        int64_t chunk_rows = 0;  // sizes the launch: the decode rows are not its
+        for (int32_t l : pre_len) chunk_rows += l;
+        int rc = prefill_batch(c, layer, pre, pre_len, pre_off, chunk_rows, q, q_dtype, q_token_stride, out, num_heads,
                                scale, mapping, ps, pre_groups);
         if (!rc)
             rc = decode_batch(c, layer, dec, nullptr, identity ? nullptr : &dec_rows, q, q_dtype, q_token_stride, out,

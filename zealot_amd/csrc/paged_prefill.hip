@@ -30,8 +30,16 @@
 //       each wave loading one page of every pair); QK^T and PV run on MFMA with
 //       a lazily rescaled softmax (see paged_decode.hip), software-pipelined
 //       one pair deep; every column carries its own visibility limit.
-// Rows write their outputs directly (no split over keys): an item reads the
-// pages up to its last row's limit, so the causal triangle costs half.
+// Rows write their outputs directly: an item reads the pages up to its last
+// row's limit, so the causal triangle costs half.
+// Small batches run prefill_mfma_kernel without the plan and the queues
+// (DIRECT), one workgroup per item, and where the items leave the chip idle
+// (one prompt's chunk behind a long context) split each over its keys;
+// prefill_reduce_kernel merges the splits.  A 389-token chunk behind 7680
+// tokens, 32 / 8 heads of 128 bf16: 167 us planned (104 workgroups on 256
+// CUs), 82 us in four splits (75 attention, bound by the CUs that hold two of
+// the 416 workgroups, 8 merge); a 20-token chunk behind 100: 17 and 15 us, host
+// time the most of it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -60,6 +68,8 @@ constexpr int kXcds = 8;                         // XCDs of an MI355X
 constexpr int kXcdBins = kMaxBins / kXcds;       // longest-first bins per XCD queue
 constexpr int kQueueStride = 32;                 // ints between XCD queue heads (128 B)
 constexpr float kRescaleSlack = 8.0f;  // lazy-rescale slack, log2 units
+constexpr float kNoKeyMax = -1e30f;    // reference max of a row that has seen no key yet
+constexpr int kMaxSplits = 16;         // key splits of a planless item
 
 struct PParams {
     const void *q;        // [T, H, D]
@@ -81,6 +91,12 @@ struct PParams {
     int64_t num_blocks;
     float scale_log2;
     int grouped, q_f32, causal;
+    // planless launches (items and work unused): pages per split, the most
+    // splits of an item, and the splits' partials: (m, l) and unnormalised rows
+    // of item slot (tile * Hkv + kvh) * splits + split, kRows rows each
+    int split_pages, splits;
+    float2 *ml;
+    float *po;
 };
 
 __device__ __forceinline__ int chunk_len(const PParams &p, int n) {
@@ -99,6 +115,46 @@ __device__ __forceinline__ int tile_pages(const PParams &p, int n, int qt) {
     const int lim = p.causal ? p.start[n] + last : p.start[n] + len;
     const int vis = min(lim, p.eff[n]);
     return (vis + p.block_size - 1) / p.block_size;
+}
+
+// A query tile of a planless launch.
+struct Tile {
+    int n, qt;      // sequence (< 0: there is none) and tile
+    int len, st;    // the sequence's chunk length and cached tokens
+    int64_t row;    // its first q row
+    int pages;      // pages the tile sees when no table entry cuts them
+};
+
+// Query tile `slot` of all sequences' tiles in order: one load round trip (a
+// sequence per lane), the rest lane reads.  Uniform over the wave; every lane
+// must call it.
+__device__ __forceinline__ Tile find_tile(const PParams &p, int slot, int lane) {
+    Tile t{-1, 0, 0, 0, 0, 0};
+    for (int n0 = 0; n0 < p.num_seqs; n0 += kWave) {
+        const int i = min(n0 + lane, p.num_seqs - 1);
+        const int len = chunk_len(p, i), st = p.start[i], row = (int)chunk_row0(p, i);
+        const int tiles = n0 + lane < p.num_seqs ? (len + p.tq - 1) / p.tq : 0;
+        int incl = tiles;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int u = __shfl_up(incl, o);
+            if (lane >= o) incl += u;
+        }
+        const uint64_t at = __builtin_amdgcn_ballot_w64(slot < incl);
+        if (at) {
+            const int j = (int)__builtin_ctzll(at);
+            t.n = n0 + j;
+            t.qt = slot - (__builtin_amdgcn_readlane(incl, j) - __builtin_amdgcn_readlane(tiles, j));
+            t.len = __builtin_amdgcn_readlane(len, j);
+            t.st = __builtin_amdgcn_readlane(st, j);
+            t.row = __builtin_amdgcn_readlane(row, j);
+            const int lim = p.causal ? t.st + min(t.len, (t.qt + 1) * p.tq) : t.st + t.len;
+            t.pages = (max(0, min(lim, p.max_blocks * p.block_size)) + p.block_size - 1) / p.block_size;
+            return t;
+        }
+        slot -= __builtin_amdgcn_readlane(incl, kWave - 1);
+    }
+    return t;
 }
 
 // At most 64 VGPRs a lane (eight waves a SIMD): in a mixed step this kernel
@@ -236,7 +292,12 @@ struct LdsVec<8> { typedef u32x2 T; };
 template <>
 struct LdsVec<4> { typedef uint32_t T; };
 
-template <int KV, int D, int G>
+// DIRECT: no plan and no queue; workgroup (kvh, tile slot, split) finds its
+// tile in the chunk lengths, takes split_pages pages of its context and ends.
+// An item of several splits leaves partials, which prefill_reduce_kernel
+// merges; a split whose pages end at an invalid table entry marks its sums
+// (sign bit of l), and the splits after it are dropped there.
+template <int KV, int D, int G, bool DIRECT>
 // At most 256 registers a lane (two waves a SIMD): the operands stay in
 // VGPRs, so the kernel uses no AGPRs.
 __global__ void __launch_bounds__(kWave * kWaves) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd)))
@@ -293,9 +354,12 @@ prefill_mfma_kernel(PParams p) {
 
     // this wave's XCD queue (round-robin dispatch); its first item is static
     const int xcd = blockIdx.x % kXcds;
-    const int32_t *myq = p.work + 64 + kQueueStride * xcd;
-    int item = myq[0] + (int)blockIdx.x / kXcds;
-    if (item >= myq[1]) item = -1;
+    int item = 0;
+    if constexpr (!DIRECT) {
+        const int32_t *myq = p.work + 64 + kQueueStride * xcd;
+        item = myq[0] + (int)blockIdx.x / kXcds;
+        if (item >= myq[1]) item = -1;
+    }
     int next = -1;
     // thread 0: next item from this XCD's queue, else from the others'
     auto claim = [&]() {
@@ -318,10 +382,35 @@ prefill_mfma_kernel(PParams p) {
     };
     if (item < 0) item = bcast(threadIdx.x == 0 ? claim() : -1);
     while (item >= 0) {
-        const int4 desc = p.items[item];
-        const int n = desc.x, qt = desc.y, np = desc.z, kvh = desc.w;
-        const int len = chunk_len(p, n), st = p.start[n], eff = p.eff[n];
-        const int64_t row0 = chunk_row0(p, n) + (int64_t)qt * p.tq;  // first q row of the item
+        int n, qt, np, kvh, eff, len, st;
+        int64_t row0;            // first q row of the item
+        int p0 = 0, nsplit = 1;  // first page of the split; splits of the item
+        bool cut = false;
+        constexpr int TL = 4;    // table entries a lane holds: a split of up to TL * 64 pages
+        int32_t ent[TL];
+        if constexpr (DIRECT) {
+            kvh = blockIdx.x;
+            const Tile t = find_tile(p, (int)(gridDim.y - 1 - blockIdx.y), lane);  // the last tiles, the longest, first
+            if (t.n < 0) return;
+            n = t.n, qt = t.qt, len = t.len, st = t.st;
+            row0 = t.row + (int64_t)qt * p.tq;
+            nsplit = max(1, (t.pages + p.split_pages - 1) / p.split_pages);
+            if ((int)blockIdx.z >= nsplit) return;
+            p0 = blockIdx.z * p.split_pages;
+            np = min(p.split_pages, t.pages - p0);
+            eff = min(max(0, st + len), p.max_blocks * BS);
+            // this split's table entries (each wave all of them), checked
+            // below, after the Q loads are on their way too
+            const int32_t *row = p.bt + (size_t)n * p.max_blocks + p0;
+#pragma unroll
+            for (int j = 0; j < TL; ++j) ent[j] = row[max(0, min(j * kWave + lane, np - 1))];
+        } else {
+            const int4 desc = p.items[item];
+            n = desc.x, qt = desc.y, np = desc.z, kvh = desc.w;
+            len = chunk_len(p, n), st = p.start[n], eff = p.eff[n];
+            row0 = chunk_row0(p, n) + (int64_t)qt * p.tq;
+        }
+        const int pos0 = p0 * BS;  // positions below are relative to the split
 
         // rows: column col of this wave's tile t is item row r = 64 w + 16 t + col
         // = token r / G, head r % G
@@ -332,8 +421,6 @@ prefill_mfma_kernel(PParams p) {
         for (int t = 0; t < T; ++t) {
             const int r = kWaveRows * w + 16 * t + col, tok = qt * p.tq + r / G;
             real[t] = tok < len;
-            const int tok_c = min(tok, len - 1);  // padding rows see what the last row sees
-            lim[t] = min(p.causal ? st + tok_c + 1 : st + len, eff);
             if (real[t]) {
                 const size_t qb = (size_t)(row0 + r / G) * (size_t)p.q_stride + (size_t)qhead_of(p, kvh, r % G, G) * D +
                                   (size_t)grp * DG;
@@ -356,12 +443,31 @@ prefill_mfma_kernel(PParams p) {
                 for (int kk = 0; kk < KK; ++kk) qf[t][kk] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
             }
         }
-        // the Q fragments are ready here (their loads' wait stays out of the
-        // page loop)
+        if constexpr (DIRECT) {  // the walk over this split's entries
+            int first_bad = np;
 #pragma unroll
-        for (int t = 0; t < T; ++t)
+            for (int j = TL - 1; j >= 0; --j) {
+                const uint64_t bad = __builtin_amdgcn_ballot_w64(j * kWave + lane < np &&
+                                                                 (ent[j] < 0 || (int64_t)ent[j] >= p.num_blocks));
+                if (bad) first_bad = j * kWave + (int)__builtin_ctzll(bad);
+            }
+            const int32_t *row = p.bt + (size_t)n * p.max_blocks + p0;
+            for (int i0 = TL * kWave; i0 < np && first_bad == np; i0 += kWave) {  // an unsplit long context
+                const int32_t b = row[min(i0 + lane, np - 1)];
+                const uint64_t bad = __builtin_amdgcn_ballot_w64(i0 + lane < np && (b < 0 || (int64_t)b >= p.num_blocks));
+                if (bad) first_bad = i0 + (int)__builtin_ctzll(bad);
+            }
+            if (first_bad < np) {
+                cut = true;
+                np = first_bad;
+                eff = (p0 + first_bad) * BS;
+            }
+        }
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[t][kk]));
+        for (int t = 0; t < T; ++t) {
+            const int tok_c = min(qt * p.tq + (kWaveRows * w + 16 * t + col) / G, len - 1);  // padding rows see what the last row sees
+            lim[t] = min(p.causal ? st + tok_c + 1 : st + len, eff) - pos0;
+        }
         float sl2 = p.scale_log2, vscale = 1.0f;
         if constexpr (KV == ZK_FP8_E4M3) {
             sl2 *= p.k_scales[(size_t)n * Hkv + kvh];
@@ -370,7 +476,7 @@ prefill_mfma_kernel(PParams p) {
         // block ids by scalar loads (a constant-space view of the table: the
         // kernel never writes it)
         typedef const __attribute__((address_space(4))) int32_t *ctab_t;
-        const ctab_t trow = (ctab_t)(p.bt + (size_t)n * p.max_blocks);
+        const ctab_t trow = (ctab_t)(p.bt + (size_t)n * p.max_blocks + p0);
         const char *kbase = p.k_pool + ((size_t)kvh * PAGE);
         const char *vbase = p.v_pool + ((size_t)kvh * PAGE);
         const size_t block_bytes = (size_t)PAGE * Hkv;
@@ -415,10 +521,10 @@ prefill_mfma_kernel(PParams p) {
         // V rows at or past vlim are zeroed: stale rows past the context and a
         // missing second page (its LDS holds another page's bytes, which may
         // not even be finite as fp8)
-        const int vlim = min(eff, np * BS);
+        const int vlim = min(eff - pos0, np * BS);
         // pairs every row sees whole: both pages below the item's first row's
         // limit (rows are token-major, limits grow with the row)
-        const int open = min(p.causal ? st + qt * p.tq + 1 : st + len, eff) / BS / 2;
+        const int open = (min(p.causal ? st + qt * p.tq + 1 : st + len, eff) - pos0) / BS / 2;
 
         // K of pair pj as MFMA A operands
         auto read_k = [&](int pj, bf16x8 (&kop)[2][KK]) {
@@ -524,9 +630,15 @@ prefill_mfma_kernel(PParams p) {
             return fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
         };
         if (npair > 0) issue(0, page_of(0));
-        if (threadIdx.x == 0) next = claim();  // overlaps the first pairs' round trip
+        if (!DIRECT && threadIdx.x == 0) next = claim();  // overlaps the first pairs' round trip
         for (int i = 1; i < min(npair, kStages - 1); ++i) issue(i, page_of(i));
         int nblk = npair > 0 ? page_of(kStages - 1) : 0;  // the next refill's page
+        // the Q fragments are ready here (their loads' wait stays out of the
+        // page loop, and behind the first pages' issue)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[t][kk]));
         // pair 0's scores set the rows' reference maxima (key 0 is visible to
         // every row, so they are finite)
         if (npair > 0) {
@@ -553,6 +665,9 @@ prefill_mfma_kernel(PParams p) {
                 float cm = lane_max(scb[0][t]) * sl2;
                 cm = fmaxf(cm, xor16(cm));
                 m[t] = fmaxf(cm, xor32(cm));
+                // a later split's first keys may all lie past a row's limit:
+                // a finite reference keeps its weights 0 and not NaN
+                if constexpr (DIRECT) m[t] = fmaxf(m[t], kNoKeyMax);
             }
         }
         // Iteration j: the weights of pair j (P) go through PV while pair
@@ -681,6 +796,26 @@ prefill_mfma_kernel(PParams p) {
             const float lt = lsum[t][0];  // the row's total (every element holds it)
             if (!real[t]) continue;
             const int r = kWaveRows * w + 16 * t + col;
+            if constexpr (DIRECT) {
+                if (nsplit > 1) {  // a partial row for the merge
+                    const size_t slot = (((size_t)(gridDim.y - 1 - blockIdx.y) * Hkv + kvh) * p.splits + blockIdx.z) * kRows + r;
+                    if (grp == 0) p.ml[slot] = make_float2(npair > 0 ? m[t] : kNoKeyMax, cut ? -lt : lt);
+                    float *po = p.po + slot * D;
+                    if constexpr (KV == ZK_BF16) {
+#pragma unroll
+                        for (int dt = 0; dt < DT; ++dt) __builtin_memcpy(po + 16 * dt + 4 * grp, &o[dt][t], 16);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float v[DT];
+#pragma unroll
+                            for (int dt = 0; dt < DT; ++dt) v[dt] = o[dt][t][i];
+                            __builtin_memcpy(po + DT * (4 * grp + i), v, sizeof(v));
+                        }
+                    }
+                    continue;
+                }
+            }
             const float inv = lt > 0.0f ? vscale / lt : 0.0f;
             const size_t ob = ((size_t)(row0 + r / G) * H + qhead_of(p, kvh, r % G, G)) * D;
             if constexpr (KV == ZK_BF16) {
@@ -714,18 +849,89 @@ prefill_mfma_kernel(PParams p) {
                 }
             }
         }
+        if constexpr (DIRECT) return;
         item = bcast(next);
     }
 }
 
+// Merges the splits of planless launches' items: workgroup (kvh, tile slot, z)
+// takes 32 of the item's kRows rows, D / 4 lanes a row, the splits' partials of
+// a row all in flight at once (S: p.splits rounded up to a power of two).
+template <int D, int G, int S>
+__global__ void __launch_bounds__(256) prefill_reduce_kernel(PParams p) {
+    constexpr int LP = D / 4, RP = 256 / LP;  // lanes per row, rows at once
+    const int lane = threadIdx.x % kWave, kvh = blockIdx.x, slot = blockIdx.y, Hkv = p.num_kv_heads;
+    const Tile tile = find_tile(p, slot, lane);
+    const int n = tile.n, qt = tile.qt, len = tile.len;
+    if (n < 0) return;
+    const int nsplit = (tile.pages + p.split_pages - 1) / p.split_pages;
+    if (nsplit <= 1) return;  // written by the attention kernel
+    const int d0 = 4 * (threadIdx.x % LP);
+    const int64_t row0 = tile.row + (int64_t)qt * p.tq;
+    const size_t base = ((size_t)slot * Hkv + kvh) * p.splits * kRows;
+    const float vscale = p.v_scales ? p.v_scales[(size_t)n * Hkv + kvh] : 1.0f;
+#pragma unroll
+    for (int k = 0; k < 32 / RP; ++k) {
+        const int r = 32 * blockIdx.z + RP * k + threadIdx.x / LP;
+        if (qt * p.tq + r / G >= len) continue;
+        float2 ml[S];
+        f32x4 x[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const size_t at = base + (size_t)(s < nsplit ? s : 0) * kRows + r;
+            ml[s] = p.ml[at];
+            x[s] = *reinterpret_cast<const f32x4 *>(p.po + at * D + d0);
+        }
+        int ns = nsplit;
+#pragma unroll
+        for (int s = S - 1; s >= 0; --s)
+            if (s < ns && (__float_as_uint(ml[s].y) >> 31)) ns = s + 1;
+        float M = kNoKeyMax, L = 0.0f;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s < ns) M = fmaxf(M, ml[s].x);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s < ns) {
+                const float wt = exp2_fast(ml[s].x - M);
+                L += fabsf(ml[s].y) * wt;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[c] = fmaf(wt, x[s][c], acc[c]);
+            }
+        const float inv = L > 0.0f ? vscale / L : 0.0f;
+        const size_t ob = ((size_t)(row0 + r / G) * p.num_heads + qhead_of(p, kvh, r % G, G)) * D + d0;
+        acc *= inv;
+        if (p.q_f32) {
+            __builtin_memcpy((float *)p.out + ob, &acc, sizeof(acc));
+        } else {
+            const uint32_t v[2] = {bf16x2_rne(acc[0], acc[1]), bf16x2_rne(acc[2], acc[3])};
+            __builtin_memcpy((uint16_t *)p.out + ob, v, sizeof(v));
+        }
+    }
+}
+
+template <int KV, int D, int G>
+void launch_k(const PParams &p, hipStream_t s) {
+    if (p.split_pages == 0) {
+        prefill_mfma_kernel<KV, D, G, false><<<p.num_groups, kWave * kWaves, 0, s>>>(p);
+        return;
+    }
+    prefill_mfma_kernel<KV, D, G, true><<<dim3(p.num_kv_heads, p.max_items, p.splits), kWave * kWaves, 0, s>>>(p);
+    const dim3 rgrid(p.num_kv_heads, p.max_items, kRows / 32);
+    if (p.splits > 8) prefill_reduce_kernel<D, G, 16><<<rgrid, 256, 0, s>>>(p);
+    else if (p.splits > 4) prefill_reduce_kernel<D, G, 8><<<rgrid, 256, 0, s>>>(p);
+    else if (p.splits > 2) prefill_reduce_kernel<D, G, 4><<<rgrid, 256, 0, s>>>(p);
+    else if (p.splits > 1) prefill_reduce_kernel<D, G, 2><<<rgrid, 256, 0, s>>>(p);
+}
+
 template <int KV, int D>
-bool launch_g(const PParams &p, hipStream_t s, int G) {
+void launch_g(const PParams &p, hipStream_t s, int G) {
     switch (G) {
-        case 1: prefill_mfma_kernel<KV, D, 1><<<p.num_groups, kWave * kWaves, 0, s>>>(p); return true;
-        case 2: prefill_mfma_kernel<KV, D, 2><<<p.num_groups, kWave * kWaves, 0, s>>>(p); return true;
-        case 4: prefill_mfma_kernel<KV, D, 4><<<p.num_groups, kWave * kWaves, 0, s>>>(p); return true;
-        case 8: prefill_mfma_kernel<KV, D, 8><<<p.num_groups, kWave * kWaves, 0, s>>>(p); return true;
-        default: return false;
+        case 1: launch_k<KV, D, 1>(p, s); break;
+        case 2: launch_k<KV, D, 2>(p, s); break;
+        case 4: launch_k<KV, D, 4>(p, s); break;
+        default: launch_k<KV, D, 8>(p, s); break;
     }
 }
 
@@ -749,12 +955,60 @@ int max_items_for(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads
     return (int)std::min<int64_t>(m, 0x3fffffff);
 }
 
+// Planless launches.  Items a batch makes, about: every sequence's last tile is
+// on average half used.
+int64_t planless_items(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads) {
+    const int tq = std::max(1, kRows / std::max(1, num_heads / num_kv_heads));
+    return std::max<int64_t>(1, ((total_q + tq - 1) / tq + num_seqs / 2) * num_kv_heads);
+}
+constexpr int64_t kFill = 512;  // workgroups that fill the chip, two a CU
+// Key splits such a launch may use: its share of the chip (fill workgroups) full
+// once.
+int max_splits_for(int64_t items, int64_t fill) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, fill / items));
+}
+// Splits of an item of up to `pages` pages, from what the parts measured (us): a
+// workgroup costs 9 besides its pairs, a pair 0.62 with one workgroup a CU and
+// about 0.8 with two (items of mixed lengths), the merge 7 and the partials'
+// traffic (67 KB each, written and read at 5 TB/s).
+int splits_for(int64_t items, int pages, int64_t fill) {
+    int best = 1;
+    double best_us = 1e30;
+    for (int s = 1; s <= max_splits_for(items, fill); ++s) {
+        const double us = (items * s <= kFill / 2 ? 0.62 : 0.8) * (pages / 2.0 / s) +
+                          (s > 1 ? 7.0 + items * s * 0.027 : 0.0);
+        if (us < best_us) {
+            best_us = us;
+            best = s;
+        }
+    }
+    return best;
+}
+// Whether a launch runs without a plan: its items start at once, or the work is
+// short (items x page pairs) against what the plan kernel costs (7-18 us in
+// front of everything).  Longest-first order and tiles of one context side by
+// side on an XCD, which the plan gives, win on more work: 4 chunks of 512 behind
+// 4000..12000 tokens 275 us planned, 290 planless, 16 chunks of 64..256 behind
+// 0..2000 77 and 57 (3 of 737, 64 heads: 101 and 78).
+// Beside a decode (a mixed step) only what fits the share does: 100 decodes and
+// 3 chunks of 300 took 133 us planned, 148 with two workgroups on every CU.
+bool planless(int64_t items, int pages, int64_t fill) {
+    return items <= fill || (fill == kFill && items <= 3 * kFill && items * (pages / 2) <= 100000);
+}
+constexpr size_t kPartBytes = (size_t)kRows * (sizeof(float2) + 128 * sizeof(float));  // an item split's partials, D <= 128
+
 int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, zk_dtype kv_dtype,
                  void *out, const int32_t *block_tables, const int64_t *cu_seqlens_q, const int64_t *q_off,
                  const int32_t *q_len, const int32_t *start_pos, int num_seqs, int64_t total_q, int num_heads,
                  int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq, int64_t num_blocks,
                  float scale, int causal, zk_gqa_mapping mapping, const float *k_scales, const float *v_scales,
                  void *workspace, size_t workspace_bytes, void *stream, int64_t q_stride, int max_groups);
+
+size_t plan_bytes(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads) {
+    return align256(sizeof(int32_t) * (size_t)num_seqs) + kWorkBytes +
+           align256(sizeof(int4) * (size_t)max_items_for(num_seqs, total_q, num_heads, num_kv_heads) *
+                    (size_t)num_kv_heads);
+}
 
 }  // namespace
 
@@ -776,10 +1030,11 @@ int zk::paged_prefill_rows(const void *q, zk_dtype q_dtype, const void *k_pool, 
 extern "C" {
 
 size_t zk_paged_prefill_workspace_size(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads) {
-    if (num_seqs <= 0 || total_q < 0) return 256;
-    return align256(sizeof(int32_t) * (size_t)num_seqs) + kWorkBytes +
-           align256(sizeof(int4) * (size_t)max_items_for(num_seqs, total_q, num_heads, num_kv_heads) *
-                    (size_t)num_kv_heads);
+    if (num_seqs <= 0 || total_q < 0 || num_heads <= 0 || num_kv_heads <= 0) return 256;
+    // the plan's, or the planless launch's partials
+    const int splits = max_splits_for(planless_items(num_seqs, total_q, num_heads, num_kv_heads), kFill);
+    const size_t slots = (size_t)max_items_for(num_seqs, total_q, num_heads, num_kv_heads) * num_kv_heads;
+    return std::max(plan_bytes(num_seqs, total_q, num_heads, num_kv_heads), splits > 1 ? slots * splits * kPartBytes : 0);
 }
 
 int zk_paged_prefill(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, zk_dtype kv_dtype,
@@ -831,7 +1086,7 @@ int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void
     if (fp8 != (k_scales != nullptr && v_scales != nullptr))
         return set_error(ZK_ERR_INVALID_ARGUMENT,
                          "Internal error: zk_paged_prefill: fp8 pools need k/v scales, other pools none");
-    const size_t need = zk_paged_prefill_workspace_size(num_seqs, total_q, num_heads, num_kv_heads);
+    const size_t need = plan_bytes(num_seqs, total_q, num_heads, num_kv_heads);
     if (workspace_bytes < need || ((uintptr_t)workspace & 255u))
         return set_error(ZK_ERR_INVALID_ARGUMENT,
                          "Internal error: zk_paged_prefill: workspace too small or not 256-B aligned (need " +
@@ -869,8 +1124,20 @@ int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void
     p.grouped = mapping == ZK_GQA_GROUPED ? 1 : 0;
     p.q_f32 = q_dtype == ZK_F32 ? 1 : 0;
     p.causal = causal ? 1 : 0;
+    p.split_pages = p.splits = 0;
+    const int64_t items = planless_items(num_seqs, total_q, num_heads, num_kv_heads);
+    const int64_t fill = max_groups > 0 ? std::min<int64_t>(max_groups, kFill) : kFill;
+    if (planless(items, max_blocks_per_seq, fill) && p.max_items <= 65535) {
+        const size_t slots = (size_t)p.max_items * num_kv_heads;
+        int splits = splits_for(items, max_blocks_per_seq, fill);
+        if (slots * splits * kPartBytes > workspace_bytes) splits = 1;
+        p.split_pages = ((max_blocks_per_seq + splits - 1) / splits + 1) / 2 * 2;  // whole page pairs
+        p.splits = (max_blocks_per_seq + p.split_pages - 1) / p.split_pages;
+        p.ml = (float2 *)ws;
+        p.po = (float *)(ws + slots * p.splits * kRows * sizeof(float2));
+    }
     hipStream_t s = (hipStream_t)stream;
-    {
+    if (p.split_pages == 0) {
         KernelTimer timer("prefill_plan", s);
         prefill_plan_kernel<<<1, 1024, 0, s>>>(p);
     }

@@ -123,7 +123,7 @@ int paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const void
 bool paged_decode_fuses_append(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
 // zk_paged_prefill with the chunk rows of sequence n given as a device
 // offset and length (q_off[n], q_len[n]) instead of cu_seqlens_q; total_q is
-// an upper bound of the rows; q rows are q_stride elements apart (0 = H * D).
+// an upper bound of the sum of the lengths; q rows are q_stride elements apart (0 = H * D).
 // max_groups > 0 caps the persistent grid (two-wave workgroups; 0: two per
 // CU, every SIMD), leaving SIMDs to a kernel that runs beside it.
 int paged_prefill_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, zk_dtype kv_dtype,
