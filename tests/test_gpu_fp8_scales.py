@@ -1,0 +1,32 @@
+"""zk_fp8_scales on the MI355X, value for value against numpy: rows of whole and
+of ragged 16-byte chunks, empty and one-token sequences, more chunks than one
+round of a workgroup's loads, all-zero heads (scale 1), NaN (ignored) and
+infinities, and a source off its 16-byte alignment."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [128, 64, 96, 100, 7])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("off", [0, 1])
+def test_scales_match_numpy(D, dtype, off):
+    from zealot_amd import ops
+    hkv, lens = 3, [0, 1, 3, 700, 64, 513]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    T = int(cu[-1])
+    store = torch.randn(T * hkv * D + off, generator=torch.Generator().manual_seed(D + off)).to(dtype)
+    x = store[off:].view(T, hkv, D)
+    x[1:4, 1] = 0.0
+    x[4 + 650, 2, D - 1] = 1000.0  # the last element of a late row
+    x[10, 0, 0] = float("nan")
+    x[-1, 0, 0] = float("-inf")
+    dev = store.cuda()[off:].view(T, hkv, D)
+    got = ops.fp8_scales(dev, torch.from_numpy(cu).cuda()).cpu().numpy()
+    a = np.abs(x.float().numpy())
+    for n, length in enumerate(lens):
+        m = np.nanmax(a[cu[n]:cu[n + 1]], axis=(0, 2)) if length else np.zeros(hkv, np.float32)
+        want = np.where(m > 0, m.astype(np.float32) / np.float32(448.0), np.float32(1.0))
+        np.testing.assert_array_equal(got[n], want)

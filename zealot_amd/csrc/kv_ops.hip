@@ -254,40 +254,62 @@ append_elem_kernel(const void *__restrict__ k, const void *__restrict__ v, void 
 }
 
 // ------------------------------------------------------------- fp8 scales
-// One workgroup per (sequence, kv head); each thread takes whole token rows
-// (head_dim values) so every lane has a row's worth of loads in flight.
-__global__ void __launch_bounds__(kThreads)
-fp8_scales_kernel(const void *__restrict__ x, int src_dt, const int64_t *__restrict__ cu,
-                  uint32_t hkv, uint32_t head_dim, float *__restrict__ scales) {
-    __shared__ float red[kThreads / 64];
+// amax over the values of one 16-byte word (NaN ignored, as fmaxf does).
+template <int SRC>
+__device__ __forceinline__ float amax16(uint4 w) {
+    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (SRC == ZK_F32) m = fmaxf(m, fabsf(__uint_as_float(ws[j])));
+        else m = fmaxf(m, fmaxf(fabsf(bf16lo(ws[j])), fabsf(bf16hi(ws[j]))));
+    }
+    return m;
+}
+
+// One workgroup per (sequence, kv head), a 1024-thread one since the sequences
+// of a prompt batch are few: the head's rows are read as one line of 16-byte
+// chunks, consecutive lanes consecutive chunks of a row, eight loads a thread in
+// flight.  Bound by what one CU can have in flight: 12 prompts of 60..2000
+// tokens, 8 heads of 128 bf16 (28 MB) 15 us (37 us with a whole row a
+// thread, whose loads touch 64 lines each).  Rows that are not 16-byte chunks
+// go element by element.
+constexpr int kScaleThreads = 1024;
+template <int SRC, bool VEC>
+__global__ void __launch_bounds__(kScaleThreads)
+fp8_scales_kernel(const void *__restrict__ x, const int64_t *__restrict__ cu, uint32_t hkv, uint32_t head_dim,
+                  float *__restrict__ scales) {
+    constexpr int U = 8;
+    constexpr uint32_t ES = SRC == ZK_F32 ? 4 : 2;
+    __shared__ float red[kScaleThreads / 64];
     const uint32_t n = blockIdx.x, h = blockIdx.y;
     const int64_t t0 = cu[n], t1 = cu[n + 1];
-    const uint32_t es = src_dt == ZK_F32 ? 4 : 2;
-    const bool vec = ((head_dim * es) % 16) == 0 && (((uintptr_t)x) & 15u) == 0;
     float amax = 0.0f;
-    for (int64_t t = t0 + threadIdx.x; t < t1; t += kThreads) {
-        const size_t off = ((size_t)t * hkv + h) * head_dim;
-        if (vec) {
-            const uint4 *row = reinterpret_cast<const uint4 *>((const char *)x + off * es);
-            const uint32_t n16 = head_dim * es / 16;
-            for (uint32_t c = 0; c < n16; ++c) {
-                const uint4 w = row[c];
-                const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    if (t1 > t0) {
+        const uint64_t per_row = VEC ? head_dim * ES / 16 : head_dim, total = (uint64_t)(t1 - t0) * per_row;
+        const char *base = (const char *)x + ((size_t)t0 * hkv + h) * head_dim * ES;
+        const size_t row_bytes = (size_t)hkv * head_dim * ES;
+        for (uint64_t i0 = threadIdx.x; i0 < total; i0 += (uint64_t)U * kScaleThreads) {
+            if constexpr (VEC) {
+                uint4 v[U];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (src_dt == ZK_F32) {
-                        amax = fmaxf(amax, fabsf(__uint_as_float(ws[j])));
-                    } else {
-                        amax = fmaxf(amax, fabsf(bf16lo(ws[j])));
-                        amax = fmaxf(amax, fabsf(bf16hi(ws[j])));
-                    }
+                for (int u = 0; u < U; ++u) {
+                    uint64_t i = i0 + (uint64_t)u * kScaleThreads;
+                    if (i >= total) i = i0;  // again: the maximum does not mind
+                    const uint64_t r = total <= 0xffffffffu ? (uint32_t)i / (uint32_t)per_row : i / per_row;
+                    v[u] = ld16(base + r * row_bytes + (i - r * per_row) * 16);
                 }
-            }
-        } else {
-            for (uint32_t d = 0; d < head_dim; ++d) {
-                const float val = src_dt == ZK_F32 ? ((const float *)x)[off + d]
-                                                   : __uint_as_float((uint32_t)((const uint16_t *)x)[off + d] << 16);
-                amax = fmaxf(amax, fabsf(val));
+#pragma unroll
+                for (int u = 0; u < U; ++u) amax = fmaxf(amax, amax16<SRC>(v[u]));
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const uint64_t i = i0 + (uint64_t)u * kScaleThreads;
+                    if (i >= total) break;
+                    const uint64_t r = i / per_row;
+                    const char *e = base + r * row_bytes + (i - r * per_row) * ES;
+                    amax = fmaxf(amax, fabsf(SRC == ZK_F32 ? *(const float *)e : __uint_as_float((uint32_t) * (const uint16_t *)e << 16)));
+                }
             }
         }
     }
@@ -296,7 +318,7 @@ fp8_scales_kernel(const void *__restrict__ x, int src_dt, const int64_t *__restr
     __syncthreads();
     if (threadIdx.x == 0) {
         float m = red[0];
-        for (int i = 1; i < kThreads / 64; ++i) m = fmaxf(m, red[i]);
+        for (int i = 1; i < kScaleThreads / 64; ++i) m = fmaxf(m, red[i]);
         scales[(size_t)n * hkv + h] = m > 0.0f ? m / 448.0f : 1.0f;
     }
 }
@@ -661,8 +683,10 @@ int zk_fp8_scales(const void *x, zk_dtype src_dtype, const int64_t *cu_seqlens, 
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_fp8_scales: NULL pointer");
     dim3 grid(num_seqs, num_kv_heads);
     KernelTimer timer("fp8_scales", (hipStream_t)stream);
-    fp8_scales_kernel<<<grid, kThreads, 0, (hipStream_t)stream>>>(x, src_dtype, cu_seqlens, num_kv_heads,
-                                                                 head_dim, scales);
+    const bool vec = ((size_t)head_dim * elt_size(src_dtype)) % 16 == 0 && ((uintptr_t)x & 15u) == 0;
+    auto kernel = src_dtype == ZK_F32 ? (vec ? fp8_scales_kernel<ZK_F32, true> : fp8_scales_kernel<ZK_F32, false>)
+                                      : (vec ? fp8_scales_kernel<ZK_BF16, true> : fp8_scales_kernel<ZK_BF16, false>);
+    kernel<<<grid, kScaleThreads, 0, (hipStream_t)stream>>>(x, cu_seqlens, num_kv_heads, head_dim, scales);
     return check_launch("zk_fp8_scales");
 }
 
