@@ -71,6 +71,16 @@ struct Plan {
     bool tiled = false;            // a plan for tiled weights (skinny kernel only)
 };
 
+// What the timing kept for decode-sized products (m <= 64): shared by every m
+// with the same number of 16-row tiles, so a batch that grows by one neither
+// times a shape again (0.4 s and more of a first call) nor draws another split
+// of k, and with it another rounding, from timings 1.5 % apart.
+struct Choice {
+    int splits, tile_rows, fused_splits, fused_rows;
+    hipblasLtMatmulAlgo_t algo;
+};
+constexpr int64_t kSharedRows = 64;
+
 // Workspaces of one stream: hipBLASLt's, and the skinny kernel's split-k
 // sums (allocated when a plan first needs them).
 struct Scratch {
@@ -85,6 +95,7 @@ struct DeviceState {
     std::map<hipStream_t, Scratch> scratch;
     uint64_t clock = 0;
     std::map<std::tuple<int64_t, int64_t, int64_t, int, int, bool>, Plan> plans;  // (m, n, k, in, out, tiled)
+    std::map<std::tuple<int64_t, int64_t, int64_t, int, int, bool>, Choice> choices;  // (16-row tiles, n, k, in, out, tiled)
 };
 
 std::mutex g_mu;
@@ -323,6 +334,30 @@ int make_plan(DeviceState &d, Scratch &sc, int64_t m, int64_t n, int64_t k, zk_d
     const bool deep = m <= 256 && n * k >= (int64_t)1 << 22;
     const Problem q{x, w, y, m, n, k, out == ZK_F32};
     const bool aligned = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
+    const auto ckey = std::make_tuple((m + 15) / 16, n, k, (int)in, (int)out, false);
+    const bool shared = tune && deep && in == ZK_BF16 && aligned && m <= kSharedRows;
+    if (shared) {
+        auto c = d.choices.find(ckey);
+        if (c != d.choices.end()) {
+            const Choice &ch = c->second;
+            const float alpha = 1.0f, beta = 0.0f;
+            hipblasLtMatmulAlgo_t algo = ch.algo;
+            size_t wsz = 0;
+            const bool same_algo = hipblaslt_ext::matmulIsAlgoSupported(d.handle, p.desc, &alpha, p.a, p.b, &beta, p.c, p.c,
+                                                                        algo, wsz) == HIPBLAS_STATUS_SUCCESS &&
+                                   wsz <= kWorkspace;
+            if (ch.splits > 0 ? skinny_fits(m, n, k, ch.tile_rows, ch.splits) : same_algo) {
+                p.splits = ch.splits;
+                p.tile_rows = ch.tile_rows;
+                p.fused_splits = ch.fused_splits;
+                p.fused_rows = ch.fused_rows;
+                p.algo = same_algo ? algo : cands[0].algo;
+                p.ws = same_algo ? wsz : cands[0].ws;
+                *res = &(d.plans[key] = p);
+                return ZK_OK;
+            }
+        }
+    }
     if (tune && deep && in == ZK_BF16 && aligned &&
         (sc.partial || hipMalloc(&sc.partial, kSkinnyPartial) == hipSuccess))
         for (int rows : kSkinnyRows)
@@ -358,6 +393,7 @@ int make_plan(DeviceState &d, Scratch &sc, int64_t m, int64_t n, int64_t k, zk_d
     }
     p.algo = cands[best_blas].algo;
     p.ws = cands[best_blas].ws;
+    if (shared) d.choices[ckey] = Choice{p.splits, p.tile_rows, p.fused_splits, p.fused_rows, p.algo};
     *res = &(d.plans[key] = p);
     return ZK_OK;
 }
@@ -383,6 +419,19 @@ int make_tiled_plan(DeviceState &d, Scratch &sc, int64_t m, int64_t n, int64_t k
     if (!sc.partial) ZK_HIP_CHECK(hipMalloc(&sc.partial, kSkinnyPartial), "zk_linear skinny workspace");
     Plan p;
     p.tiled = true;
+    const auto ckey = std::make_tuple((m + 15) / 16, n, k, (int)ZK_BF16, (int)out, true);
+    const bool shared = tune && m <= kSharedRows;
+    if (shared) {
+        auto c = d.choices.find(ckey);
+        if (c != d.choices.end() && skinny_fits(m, n, k, c->second.tile_rows, c->second.splits, true)) {
+            p.splits = c->second.splits;
+            p.tile_rows = c->second.tile_rows;
+            p.fused_splits = c->second.fused_splits;
+            p.fused_rows = c->second.fused_rows;
+            *res = &(d.plans[key] = p);
+            return ZK_OK;
+        }
+    }
     int best = 0, best_blas = -1, best_split = -1;
     if (tune && cands.size() > 1) {
         Problem q{x, w, y, m, n, k, out == ZK_F32, true};
@@ -395,6 +444,7 @@ int make_tiled_plan(DeviceState &d, Scratch &sc, int64_t m, int64_t n, int64_t k
         p.fused_splits = cands[best_split].splits;
         p.fused_rows = cands[best_split].tile_rows;
     }
+    if (shared) d.choices[ckey] = Choice{p.splits, p.tile_rows, p.fused_splits, p.fused_rows, {}};
     *res = &(d.plans[key] = p);
     return ZK_OK;
 }
