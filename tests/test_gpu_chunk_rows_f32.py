@@ -1,0 +1,65 @@
+"""Prompt chunks on f32 pools (KVCache.attention_batch): row groups of 32 / G
+tokens on the f32 MFMA, on the MI355X against float64 attention of the same
+K / V: chunk lengths around a group, contexts of one and of several partitions,
+chunks beside decodes, both mappings, head counts and sizes, bf16 queries,
+strided and unaligned queries (the latter take the per-row decodes).  Tolerance
+1e-5 absolute (f32), 2e-2 for bf16 outputs."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(q, k, v, heads, hkv, mapping, start):
+    t, _, d = q.shape
+    g = heads // hkv
+    out = torch.empty(q.shape, dtype=torch.float64)
+    see = torch.arange(k.shape[0])[None] <= start + torch.arange(t)[:, None]
+    for h in range(heads):
+        kv = h // g if mapping == "grouped" else h % hkv
+        w = (q[:, h].double() @ k[:, kv].double().T / math.sqrt(d)).masked_fill(~see, float("-inf"))
+        out[:, h] = torch.softmax(w, 1) @ v[:, kv].double()
+    return out
+
+
+@pytest.mark.parametrize("H,Hkv,D,mapping,qdt", [(32, 8, 128, "grouped", torch.float32), (4, 4, 128, "grouped", torch.float32),
+                                                 (4, 2, 64, "modulo", torch.float32), (16, 2, 64, "grouped", torch.float32),
+                                                 (16, 2, 128, "modulo", torch.bfloat16)])
+@pytest.mark.parametrize("layout", ["packed", "strided", "unaligned"])
+def test_chunks_match_float64(H, Hkv, D, mapping, qdt, layout):
+    from zealot_amd import BlockManager, KVCache
+    nt = 32 * Hkv // H
+    n = [1, nt - 1 or 2, nt, nt + 1, 3 * nt + 2, 1, 40, 2]
+    before = [300, 0, 15, 16, 130, 0, 1000, 511]
+    total = [a + b for a, b in zip(n, before)]
+    bm = BlockManager(400, 16)
+    cache = KVCache(400, 16, 2, Hkv, D, dtype=torch.float32, max_seqs=8, max_blocks_per_seq=80)
+    g = torch.Generator().manual_seed(H + D)
+    ids = [f"s{i}" for i in range(len(n))]
+    kv = [(torch.randn(t, Hkv, D, generator=g), torch.randn(t, Hkv, D, generator=g)) for t in total]
+    for sid, t in zip(ids, total):
+        cache.register_seq(sid, 80)
+        for _ in range(-(-t // 16)):
+            cache.alloc_block(sid, bm)
+    for part in (0, 1):  # the cached tokens, then the step's
+        lens = before if part == 0 else n
+        rows = [[x[:b] if part == 0 else x[b:] for x in p] for p, b in zip(kv, before)]
+        k, v = (torch.cat([r[j] for r in rows]).cuda() for j in (0, 1))
+        for layer in ((0, 1) if part == 0 else (0,)):
+            cache.write_batch(layer, ids, lens, k, v)
+    q = torch.randn(sum(n), H, D, generator=g).to(qdt)
+    if layout == "packed":
+        qd = q.cuda()
+    else:  # rows inside a wider buffer, one element off for "unaligned"
+        off = 1 if layout == "unaligned" else 4 * D
+        buf = torch.zeros(sum(n), H * D + 8 * D, dtype=qdt, device="cuda")
+        qd = buf[:, off:off + H * D].view(sum(n), H, D)
+        qd.copy_(q)
+    got = cache.attention_batch(0, ids, n, qd, mapping=mapping).cpu().double()
+    row = 0
+    for (k, v), t, b in zip(kv, n, before):
+        want = _ref(q[row:row + t], k, v, H, Hkv, mapping, b)
+        assert (got[row:row + t] - want).abs().max() <= (1e-5 if qdt == torch.float32 else 2e-2)
+        row += t

@@ -1354,6 +1354,47 @@ int prefill_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState
                                   launch, q_stride, max_groups);
 }
 
+// The chunk rows of an f32 cache through zk::paged_rows, 32 / G tokens a group:
+// every page is read once per group (as decodes, once per row) and the tables
+// and groups have a buffer of their own, so that the decode half's uploads stay
+// valid from layer to layer.
+int chunk_rows_f32(zk_kv_cache *c, size_t layer, const std::vector<const SeqState *> &seqs,
+                   const std::vector<int32_t> &len, const std::vector<int64_t> &off, const void *q, zk_dtype q_dtype,
+                   int64_t q_stride, void *out, int num_heads, float scale, zk_gqa_mapping mapping) {
+    const size_t n = seqs.size();
+    const int nt = 32 / (num_heads / (int)c->num_kv_heads);
+    size_t stride = 1, groups = 0;
+    for (size_t i = 0; i < n; ++i) {
+        stride = std::max(stride, seqs[i]->handles.size());
+        groups += ((size_t)len[i] + nt - 1) / nt;
+    }
+    const size_t tbl_bytes = (n * stride * sizeof(int32_t) + 255) & ~(size_t)255;
+    std::vector<char> host(tbl_bytes + groups * sizeof(int4), 0);
+    int32_t *tbl = (int32_t *)host.data();
+    int4 *g = (int4 *)(host.data() + tbl_bytes);
+    for (size_t i = 0; i < n; ++i) {
+        for (size_t j = 0; j < stride; ++j)
+            tbl[i * stride + j] = j < seqs[i]->handles.size() ? (int32_t)seqs[i]->handles[j].block_id : -1;
+        const int32_t start = (int32_t)seqs[i]->layer_len[layer] - len[i];
+        for (int32_t t = 0; t < len[i]; t += nt)
+            *g++ = make_int4((int)i, (int)(off[i] + t), std::min(nt, len[i] - t), start + t + 1);
+    }
+    if (int rc = put(c, c->d_pre, host.data(), host.size(), "KVCache chunk rows")) return rc;
+    // groups of one launch: its grid's limit
+    for (size_t g0 = 0; g0 < groups; g0 += 65535) {
+        const int gn = (int)std::min<size_t>(65535, groups - g0);
+        const size_t ws = zk::paged_rows_workspace(gn, num_heads, (int)c->num_kv_heads, (int)c->head_dim, (int)stride);
+        if (int rc = c->d_pws.ensure(ws, "KVCache chunk rows workspace")) return rc;
+        char *d = (char *)c->d_pre.dev.p;
+        if (int rc = zk::paged_rows(q, q_dtype, c->k_pool(layer), c->v_pool(layer), out, (const int32_t *)d,
+                                    (const int4 *)(d + tbl_bytes) + g0, gn, num_heads, (int)c->num_kv_heads,
+                                    (int)c->head_dim, (int)stride, (int64_t)c->num_blocks, scale, mapping, c->d_pws.p,
+                                    c->d_pws.cap, c->stream, q_stride))
+            return rc;
+    }
+    return ZK_OK;
+}
+
 int ensure_side_stream(zk_kv_cache *c) {
     if (c->side) return ZK_OK;
     ZK_HIP_CHECK(hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming), "KVCache side stream");
@@ -1481,7 +1522,11 @@ int zk_cache_attention_batch(zk_kv_cache *c, size_t layer, const char *const *id
                               num_heads, scale, mapping, true))
         return rc;
     if (pre.empty()) return ZK_OK;
-    // shapes without the MFMA prefill: every chunk row is a decode of its
+    const int64_t stride_elems = q_token_stride > 0 ? q_token_stride : (int64_t)num_heads * (int64_t)c->head_dim;
+    if (zk::paged_rows_supported(c->dtype, (int)c->head_dim, (int)c->block_size, num_heads, (int)c->num_kv_heads) &&
+        (((uintptr_t)q | (uintptr_t)out) & 15u) == 0 && stride_elems % 4 == 0)
+        return chunk_rows_f32(c, layer, pre, pre_len, pre_off, q, q_dtype, q_token_stride, out, num_heads, scale, mapping);
+    // other shapes without the MFMA prefill: every chunk row is a decode of its
     // causal context (start + t + 1 tokens)
     std::vector<const SeqState *> ex;
     std::vector<int32_t> ex_len, ex_rows;

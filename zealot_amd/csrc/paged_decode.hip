@@ -138,9 +138,18 @@ struct Params {
     float scale_log2;  // softmax scale * log2(e)
     int grouped;       // 1: kv = h / G, 0: kv = h % Hkv
     int q_f32;         // Q / out dtype: 1 f32, 0 bf16
+    // Chunk rows (RowGroups in zk_common.h; null otherwise): "sequence" n of the
+    // partials and of the reduce is token n % (32 / G) of group n / (32 / G).
+    const int4 *groups;
 };
 
-__device__ __forceinline__ size_t qrow(const Params &p, int n) { return p.q_rows ? (size_t)p.q_rows[n] : (size_t)n; }
+// Tokens of a row group: its tile of 32 rows holds the G heads of each.
+__device__ __forceinline__ int group_tokens(const Params &p) { return 32 * p.num_kv_heads / p.num_heads; }
+
+__device__ __forceinline__ size_t qrow(const Params &p, int n) {
+    if (p.groups) return (size_t)p.groups[n / group_tokens(p)].y + n % group_tokens(p);
+    return p.q_rows ? (size_t)p.q_rows[n] : (size_t)n;
+}
 
 __device__ __forceinline__ int qhead_of(const Params &p, int kvh, int j, int G) {
     return p.grouped ? kvh * G + j : kvh + j * p.num_kv_heads;
@@ -169,7 +178,14 @@ __device__ __forceinline__ int shared_parts_of(const Params &p, int n) {
 // PLANLESS launches have no eff_len: the length is the caller's.
 template <bool PLANLESS = false>
 __device__ __forceinline__ int private_parts_of(const Params &p, int n) {
-    const int len = PLANLESS ? min(max(p.seq_lens[n], 0), p.max_blocks * p.block_size) : p.eff_len[n];
+    int len;
+    if (PLANLESS && p.groups) {
+        const int4 g = p.groups[n / group_tokens(p)];
+        const int i = n % group_tokens(p);
+        len = i < g.z ? g.w + i : 0;  // 0: no such token
+    } else {
+        len = PLANLESS ? min(max(p.seq_lens[n], 0), p.max_blocks * p.block_size) : p.eff_len[n];
+    }
     const int pages = (len + p.block_size - 1) / p.block_size;
     const int rest = pages - prefix_pages_of(p, n);
     return rest > 0 ? (rest + p.part_pages - 1) / p.part_pages : 0;
@@ -409,10 +425,18 @@ struct LdsVec<4> { typedef uint32_t T; };
 // and the table itself and ends.  A partition whose pages end at an invalid
 // table entry marks its partial (sign bit of l), and the reduce drops the
 // partitions after it.
-template <int KV, int D, int G, bool DIRECT>
+// ROWS (with DIRECT): workgroup (kvh, part, g) is partition `part` of row group g,
+// up to 32 / G consecutive tokens of one chunk: their 32 (token, head) rows are
+// two tiles, every page is read once for all of them, and each row masks the
+// tokens past its own position.  f32 pools only; bound by the f32 MFMA (128 of
+// 32 cycles a page, 1.7 us, against 0.85 for one row tile).  A 150-token chunk
+// behind 0..600 tokens, 32 / 8 heads of 128: 57 us as 150 one-row decodes, 31
+// here, and its tables no longer displace the decode half's (four uploads of a
+// step gone): the step of it and 12 decodes 113 -> 60 us.
+template <int KV, int D, int G, bool DIRECT, bool ROWS = false>
 __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     constexpr int BS = 16;
-    constexpr int BIDS = DIRECT ? kDirectPages : kMaxItemPages;
+    constexpr int BIDS = DIRECT && !ROWS ? kDirectPages : kMaxItemPages;
     constexpr bool F32 = KV == ZK_F32;
     constexpr int ELT = F32 ? 4 : KV == ZK_BF16 ? 2 : 1;
     constexpr int DG = D / 4;            // head dims per lane group in QK
@@ -602,7 +626,9 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     auto q_row = [&](int n) -> size_t { return p.q_rows ? (size_t)((cint_t)p.q_rows)[n] : (size_t)n; };
 
     // Attention of T tiles of query rows (qf) over pages [page0, page0 + np)
-    // of table `trow` for kv-head kvh; tokens at positions >= len are masked.
+    // of table `trow` for kv-head kvh; tokens at positions >= row_len[t] are
+    // masked for this lane's row of tile t, and V rows at or past len (the
+    // longest) are zeroed.
     // trow points at the table entry of page page0; blk0 holds the block ids
     // of the first kDescPages pages.
     // Leaves O^T (o), the rows' reference max (m) and sum (l, all 4 lane
@@ -612,7 +638,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     // written into the page's LDS copy once that has landed, and to the pools
     // at byte offset row_dst of the K / V pool.
     auto attend = [&]<int T>(const qfrag_t (&qf)[T][KK], const int32_t *trow, int4 blk0, int page0, int np, int len,
-                             int kvh, float sl2, f32x4 (&o)[DT][T], float (&m)[T], float (&l)[T], int fuse_tib,
+                             const int (&row_len)[T], int kvh, float sl2, f32x4 (&o)[DT][T], float (&m)[T], float (&l)[T], int fuse_tib,
                              u32x4 nrow, size_t row_dst) {
         const char *kbase = p.k_pool + ((size_t)kvh * PAGE);
         const char *vbase = p.v_pool + ((size_t)kvh * PAGE);
@@ -756,7 +782,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             for (int t = 0; t < T; ++t) {
                 float sc[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) sc[i] = tok0 + i < len ? sacc[t][i] * sl2 : -INFINITY;
+                for (int i = 0; i < 4; ++i) sc[i] = tok0 + i < row_len[t] ? sacc[t][i] * sl2 : -INFINITY;
                 const float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
                 // lazy rescale (wave-uniform branch): the new reference is the
                 // row max over the page's 16 tokens (all four lane groups)
@@ -875,8 +901,9 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             }
         }
         f32x4 o[DT][1];
+        const int own_len[1] = {len};
         float m[1], l[1];
-        attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, kvh, sl2,
+        attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, own_len, kvh, sl2,
                                       o, m, l, fuse_tib, nrow, row_dst);
         if (col < G) {
             if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
@@ -913,7 +940,69 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         }
     };
 
-    if constexpr (DIRECT) {
+    if constexpr (ROWS) {
+        constexpr int NT = 32 / G;  // tokens of a group
+        const int kvh = blockIdx.x, part = blockIdx.y, g = blockIdx.z;
+        const int page0 = part * p.part_pages;
+        const cint_t gd = (cint_t)(p.groups + g);
+        const int4 d = make_int4(gd[0], gd[1], gd[2], gd[3]);
+        const int len = d.w + d.z - 1;  // the longest row's
+        const int want = min(p.part_pages, (len + BS - 1) / BS - page0);
+        if (want <= 0) return;
+        const int32_t *row = p.bt + (size_t)d.x * p.max_blocks + page0;
+        int np = want;  // (the caller's tables are valid up to every length; an id outside the pool still ends the walk)
+        int4 first = make_int4(0, 0, 0, 0);
+        for (int i0 = 0; i0 < want && np == want; i0 += kWave) {
+            const int e = row[min(i0 + lane, want - 1)];
+            const uint64_t bad = __builtin_amdgcn_ballot_w64(i0 + lane < want && (e < 0 || (int64_t)e >= p.num_blocks));
+            if (bad) np = i0 + (int)__builtin_ctzll(bad);
+            bids[i0 + lane] = e;
+            if (i0 == 0)
+                first = make_int4(__builtin_amdgcn_readlane(e, 0), __builtin_amdgcn_readlane(e, 1),
+                                  __builtin_amdgcn_readlane(e, 2), __builtin_amdgcn_readlane(e, 3));
+        }
+        wait_lgkmcnt0();  // visible to this wave's own reads
+        qfrag_t qf[2][KK];
+        int row_len[2];  // context of this lane's row of tile t; 0: no row
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int r = 16 * t + col;
+            row_len[t] = r / G < d.z ? d.w + r / G : 0;
+            if (row_len[t] > 0) load_q((size_t)d.y + r / G, qhead_of(p, kvh, r % G, G), qf[t]);
+            else
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) qf[t][kk] = qzero;
+        }
+        f32x4 o[DT][2];
+        float m[2], l[2];
+        attend.template operator()<2>(qf, row, first, page0, np, len, row_len, kvh, p.scale_log2, o, m, l, -1, no_row, 0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int r = 16 * t + col, qh = qhead_of(p, kvh, r % G, G);
+            const int parts = ((row_len[t] + BS - 1) / BS + p.part_pages - 1) / p.part_pages;
+            if (part >= parts) continue;  // no row, or none of its tokens here
+            if (parts > 1) {
+                store_partial(((size_t)(g * NT + r / G) * H + qh) * p.max_parts + part, o, t, 1.0f, m[t], l[t]);
+                continue;
+            }
+            const float inv = l[t] > 0.0f ? 1.0f / l[t] : 0.0f;
+            const size_t ob = ((size_t)(d.y + r / G) * H + qh) * D;
+            if (p.q_f32) {
+                store_row_f32((float *)p.out + ob, o, t, inv);
+            } else {
+#pragma unroll
+                for (int h = 0; h < DT / 4; ++h)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t v[2] = {bf16x2_rne(o[4 * h][t][i] * inv, o[4 * h + 1][t][i] * inv),
+                                               bf16x2_rne(o[4 * h + 2][t][i] * inv, o[4 * h + 3][t][i] * inv)};
+                        __builtin_memcpy((uint16_t *)p.out + ob + 64 * h + 16 * grp + 4 * i, v, 8);
+                    }
+            }
+        }
+        return;
+    }
+    if constexpr (DIRECT && !ROWS) {
         const int kvh = blockIdx.x, part = blockIdx.y, n = blockIdx.z;
         const int page0 = part * p.part_pages;
         const int32_t *row = p.bt + (size_t)n * p.max_blocks;
@@ -969,7 +1058,8 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             }
             f32x4 o[DT][2];
             float m[2], l[2];
-            attend.template operator()<2>(qf, p.bt + (size_t)n0 * p.max_blocks + page0, d1, page0, np, 0x7fffffff,
+            const int all[2] = {0x7fffffff, 0x7fffffff};
+            attend.template operator()<2>(qf, p.bt + (size_t)n0 * p.max_blocks + page0, d1, page0, np, 0x7fffffff, all,
                                           kvh, p.scale_log2, o, m, l, -1, no_row, 0);
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -1493,10 +1583,34 @@ void launch_mfma(const Params &p, hipStream_t s, int G) {
     else launch_mfma_g<KV, 64>(p, s, G);
 }
 
+// Partitions from which one workgroup a q-head merges them: eight lines of a
+// wave's loads in flight instead of a serial walk (2 sequences of 125
+// partitions: 35 -> 5 us).
+constexpr int kManyParts = 16;
+
 template <int G>
-void launch_reduce_kv(const Params &p, dim3 grid, hipStream_t s) {
-    if (p.eff_len) decode_reduce_kv_kernel<128, G, false><<<grid, kWave, 0, s>>>(p);
-    else decode_reduce_kv_kernel<128, G, true><<<grid, kWave, 0, s>>>(p);
+void launch_reduce_kv(const Params &p, bool planless, hipStream_t s) {
+    const dim3 grid(p.num_kv_heads, p.num_seqs);
+    if (planless) decode_reduce_kv_kernel<128, G, true><<<grid, kWave, 0, s>>>(p);
+    else decode_reduce_kv_kernel<128, G, false><<<grid, kWave, 0, s>>>(p);
+}
+
+// The merge for head_dim 64 or 128 (planless: partials may be marked).
+void launch_reduce(const Params &p, int G, bool planless, hipStream_t s) {
+    const dim3 rgrid(p.num_heads, p.num_seqs);
+    const bool kv = p.head_dim == 128 && (G == 2 || G == 4 || G == 8);
+    if ((planless && !kv) || p.max_parts > kManyParts) {
+        if (p.head_dim == 128) decode_reduce_many_kernel<128><<<rgrid, 256, 0, s>>>(p);
+        else decode_reduce_many_kernel<64><<<rgrid, 256, 0, s>>>(p);
+    } else if (kv) {
+        if (G == 4) launch_reduce_kv<4>(p, planless, s);
+        else if (G == 8) launch_reduce_kv<8>(p, planless, s);
+        else launch_reduce_kv<2>(p, planless, s);
+    } else if (p.head_dim == 128) {
+        decode_reduce_vec_kernel<128><<<rgrid, kWave, 0, s>>>(p);
+    } else {
+        decode_reduce_vec_kernel<64><<<rgrid, kWave, 0, s>>>(p);
+    }
 }
 
 bool mfma_supported(int kv_dtype, int head_dim, int block_size, int G) {
@@ -1509,6 +1623,23 @@ int check_launch(const char *what) {
     if (e != hipSuccess)
         return set_error(ZK_ERR_HIP, std::string("Internal error: ") + what + ": " + hipGetErrorString(e));
     return ZK_OK;
+}
+
+// Pages per shared-prefix item: about one item per two waves over all
+// subgroups' pages, so half the waves stream the shared pages (two query-row
+// tiles each) while the rest run the sequences' own items; measured best on
+// forked-prefix batches.  ZEALOT_DECODE_SHARED_PART_PAGES (16..1024) overrides.
+int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves) {
+    static const int env = [] {
+        const char *e = std::getenv("ZEALOT_DECODE_SHARED_PART_PAGES");
+        const int v = e ? std::atoi(e) : 0;
+        return v <= 0 ? 0 : (v < 16 ? 16 : (v > kMaxItemPages ? kMaxItemPages : v));
+    }();
+    if (env) return env;
+    const long half = waves / 2;
+    long pp = (total_shared_pages * num_kv_heads + half - 1) / half;
+    pp = (pp + 15) / 16 * 16;
+    return (int)(pp < 16 ? 16 : (pp > kMaxItemPages ? kMaxItemPages : pp));
 }
 
 // Planless launches: partitions of a sequence for `units` (capacity) pages
@@ -1535,28 +1666,6 @@ int direct_parts(double units, double page_bytes, int max_blocks) {
     if (bytes > kDirectBytes) return 0;
     const double pp = std::min((double)kDirectPages, std::max(8.0, std::sqrt(bytes) * 1e-3));
     return std::max((max_blocks + kDirectPages - 1) / kDirectPages, std::max(1, (int)(max_blocks / pp + 0.5)));
-}
-
-// Partitions from which one workgroup a q-head merges them: eight lines of a
-// wave's loads in flight instead of a serial walk (2 sequences of 125
-// partitions: 35 -> 5 us).
-constexpr int kManyParts = 16;
-
-// Pages per shared-prefix item: about one item per two waves over all
-// subgroups' pages, so half the waves stream the shared pages (two query-row
-// tiles each) while the rest run the sequences' own items; measured best on
-// forked-prefix batches.  ZEALOT_DECODE_SHARED_PART_PAGES (16..1024) overrides.
-int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves) {
-    static const int env = [] {
-        const char *e = std::getenv("ZEALOT_DECODE_SHARED_PART_PAGES");
-        const int v = e ? std::atoi(e) : 0;
-        return v <= 0 ? 0 : (v < 16 ? 16 : (v > kMaxItemPages ? kMaxItemPages : v));
-    }();
-    if (env) return env;
-    const long half = waves / 2;
-    long pp = (total_shared_pages * num_kv_heads + half - 1) / half;
-    pp = (pp + 15) / 16 * 16;
-    return (int)(pp < 16 ? 16 : (pp > kMaxItemPages ? kMaxItemPages : pp));
 }
 
 }  // namespace
@@ -1780,21 +1889,109 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
     }
     if (int rc = check_launch("zk_paged_decode partials")) return rc;
     if (reduce) {
-        dim3 rgrid(num_heads, num_seqs);
         KernelTimer timer("decode_reduce", s);
-        const dim3 kgrid(num_kv_heads, num_seqs);
-        const bool kv_reduce = head_dim == 128 && (G == 2 || G == 4 || G == 8);
-        if (use_mfma && ((ds.direct && !kv_reduce) || max_parts > kManyParts)) {
-            if (head_dim == 128) decode_reduce_many_kernel<128><<<rgrid, 256, 0, s>>>(p);
-            else decode_reduce_many_kernel<64><<<rgrid, 256, 0, s>>>(p);
-        } else if (head_dim == 128 && G == 4) launch_reduce_kv<4>(p, kgrid, s);
-        else if (head_dim == 128 && G == 8) launch_reduce_kv<8>(p, kgrid, s);
-        else if (head_dim == 128 && G == 2) launch_reduce_kv<2>(p, kgrid, s);
-        else if (head_dim == 128) decode_reduce_vec_kernel<128><<<rgrid, kWave, 0, s>>>(p);
-        else if (head_dim == 64) decode_reduce_vec_kernel<64><<<rgrid, kWave, 0, s>>>(p);
-        else if (head_dim == 256) decode_reduce_vec_kernel<256><<<rgrid, kWave, 0, s>>>(p);
-        else decode_reduce_kernel<<<rgrid, kWave, 0, s>>>(p);
+        if (use_mfma) {
+            launch_reduce(p, G, ds.direct, s);
+        } else {
+            const dim3 rgrid(num_heads, num_seqs);
+            if (head_dim == 128 && (G == 2 || G == 4 || G == 8)) launch_reduce(p, G, false, s);
+            else if (head_dim == 128) decode_reduce_vec_kernel<128><<<rgrid, kWave, 0, s>>>(p);
+            else if (head_dim == 64) decode_reduce_vec_kernel<64><<<rgrid, kWave, 0, s>>>(p);
+            else if (head_dim == 256) decode_reduce_vec_kernel<256><<<rgrid, kWave, 0, s>>>(p);
+            else decode_reduce_kernel<<<rgrid, kWave, 0, s>>>(p);
+        }
         if (int rc = check_launch("zk_paged_decode reduce")) return rc;
+    }
+    return ZK_OK;
+}
+
+// ------------------------------------------------------------ chunk rows on f32 pools
+bool zk::paged_rows_supported(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads) {
+    return kv_dtype == ZK_F32 && num_kv_heads > 0 && num_heads % num_kv_heads == 0 &&
+           mfma_supported(kv_dtype, head_dim, block_size, num_heads / num_kv_heads);
+}
+
+namespace {
+
+// Partitions of a group's pages: two waves a SIMD over all groups.  Of at least
+// 4 pages while the merge reads them in one round (eight partials), else of 8
+// (a partial row costs as much as two of its pages), and not 9 to 16 of them,
+// which the merge would walk one by one (150 rows behind 600 tokens: 11
+// partitions 61 us a step, 5 partitions 51).
+int rows_parts(long groups, int num_kv_heads, int max_blocks) {
+    const long want = std::max<long>(1, 2048 / std::max<long>(1, groups * num_kv_heads));
+    long parts = std::min<long>(want, max_blocks / 4);
+    if (parts > 8) {
+        parts = std::min<long>(want, max_blocks / 8);
+        if (parts <= kManyParts) parts = std::min<long>(parts, 8);
+    }
+    return (int)std::max<long>(std::max<long>(1, parts), (max_blocks + kMaxItemPages - 1) / kMaxItemPages);
+}
+WsLayout rows_layout(int groups, int num_heads, int num_kv_heads, int head_dim, int max_blocks) {
+    return ws_layout(groups * (32 * num_kv_heads / num_heads), num_heads, head_dim, rows_parts(groups, num_kv_heads, max_blocks));
+}
+
+template <int D>
+void launch_rows(const Params &p, int groups, hipStream_t s, int G) {
+    const dim3 grid(p.num_kv_heads, p.max_parts, groups);
+    switch (G) {
+        case 1: decode_mfma_kernel<ZK_F32, D, 1, true, true><<<grid, kWave, 0, s>>>(p); break;
+        case 2: decode_mfma_kernel<ZK_F32, D, 2, true, true><<<grid, kWave, 0, s>>>(p); break;
+        case 4: decode_mfma_kernel<ZK_F32, D, 4, true, true><<<grid, kWave, 0, s>>>(p); break;
+        default: decode_mfma_kernel<ZK_F32, D, 8, true, true><<<grid, kWave, 0, s>>>(p); break;
+    }
+}
+
+}  // namespace
+
+size_t zk::paged_rows_workspace(int groups, int num_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq) {
+    return rows_layout(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq).total;
+}
+
+int zk::paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, void *out,
+                   const int32_t *block_tables, const int4 *row_groups, int groups, int num_heads, int num_kv_heads,
+                   int head_dim, int max_blocks_per_seq, int64_t num_blocks, float scale, zk_gqa_mapping mapping,
+                   void *workspace, size_t workspace_bytes, void *stream, int64_t q_stride) {
+    if (groups <= 0) return ZK_OK;
+    const WsLayout w = rows_layout(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq);
+    if (groups > 65535 || workspace_bytes < w.total || ((uintptr_t)workspace & 255u))
+        return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged rows: too many groups or workspace too small");
+    const int G = num_heads / num_kv_heads;
+    Params p{};
+    p.q = q;
+    p.k_pool = (const char *)k_pool;
+    p.v_pool = (const char *)v_pool;
+    p.out = out;
+    p.bt = block_tables;
+    p.groups = row_groups;
+    p.q_stride = q_stride > 0 ? q_stride : (int64_t)num_heads * head_dim;
+    char *ws = (char *)workspace;
+    p.ml = (float2 *)(ws + w.ml);
+    p.po = (float *)(ws + w.po);
+    p.num_seqs = groups * (32 / G);
+    p.num_heads = num_heads;
+    p.num_kv_heads = num_kv_heads;
+    p.head_dim = head_dim;
+    p.block_size = 16;
+    p.max_blocks = max_blocks_per_seq;
+    p.max_parts = rows_parts(groups, num_kv_heads, max_blocks_per_seq);
+    p.part_pages = (max_blocks_per_seq + p.max_parts - 1) / p.max_parts;
+    p.num_blocks = num_blocks;
+    p.shared_part_pages = 1;
+    p.scale_log2 = scale * kLog2e;
+    p.grouped = mapping == ZK_GQA_GROUPED ? 1 : 0;
+    p.q_f32 = q_dtype == ZK_F32 ? 1 : 0;
+    hipStream_t s = (hipStream_t)stream;
+    {
+        KernelTimer timer("prefill_attention", s);
+        if (head_dim == 128) launch_rows<128>(p, groups, s, G);
+        else launch_rows<64>(p, groups, s, G);
+    }
+    if (int rc = check_launch("paged rows")) return rc;
+    if (p.max_parts > 1) {
+        KernelTimer timer("decode_reduce", s);
+        launch_reduce(p, G, /*planless=*/true, s);
+        if (int rc = check_launch("paged rows reduce")) return rc;
     }
     return ZK_OK;
 }

@@ -119,6 +119,16 @@ int paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const void
                  void *workspace, size_t workspace_bytes, void *stream, const PrefixGroups *pg,
                  const int32_t *q_rows, int64_t q_stride = 0, bool trusted_tables = false, bool reuse_plan = false,
                  const AppendRows *append = nullptr, int *head_set = nullptr, int max_waves = 0);
+// Attention of prompt-chunk rows on f32 pools (the shapes paged_rows_supported
+// names; 16-byte aligned operands): row group g = {row of block_tables, first q
+// row, tokens (at most 32 / G), context of its first token}; token i attends its
+// first w + i tokens.  Tables must be valid up to every length.
+bool paged_rows_supported(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
+size_t paged_rows_workspace(int groups, int num_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq);
+int paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, void *out,
+               const int32_t *block_tables, const int4 *row_groups, int groups, int num_heads, int num_kv_heads,
+               int head_dim, int max_blocks_per_seq, int64_t num_blocks, float scale, zk_gqa_mapping mapping,
+               void *workspace, size_t workspace_bytes, void *stream, int64_t q_stride);
 // Whether paged_decode can take a fused append for this shape.
 bool paged_decode_fuses_append(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
 // zk_paged_prefill with the chunk rows of sequence n given as a device
