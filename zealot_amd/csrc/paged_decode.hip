@@ -1599,7 +1599,8 @@ void launch_reduce_kv(const Params &p, bool planless, hipStream_t s) {
 void launch_reduce(const Params &p, int G, bool planless, hipStream_t s) {
     const dim3 rgrid(p.num_heads, p.num_seqs);
     const bool kv = p.head_dim == 128 && (G == 2 || G == 4 || G == 8);
-    if ((planless && !kv) || p.max_parts > kManyParts) {
+    // (with shared prefixes max_parts is the stride of the slots, not their number)
+    if ((planless && !kv) || (p.max_parts > kManyParts && p.num_sg == 0)) {
         if (p.head_dim == 128) decode_reduce_many_kernel<128><<<rgrid, 256, 0, s>>>(p);
         else decode_reduce_many_kernel<64><<<rgrid, 256, 0, s>>>(p);
     } else if (kv) {
