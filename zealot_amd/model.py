@@ -120,11 +120,12 @@ class HipModelRunner:
         plan = self.kv.begin_step(out)
         if not out.batch:
             return torch.empty((0, self.cfg.vocab_size), dtype=torch.float32, device=self.w.embedding.device)
+        # ids and last rows in one upload from pinned memory: the host does not
+        # wait for it, so the layers' calls run ahead of the device
         ids = [t for e in out.batch for t in e.step_input()]
-        dev = self.w.embedding.device
-        ids_dev = torch.tensor(ids, dtype=torch.int64, device=dev)
-        last = torch.tensor(plan_last_rows(plan), dtype=torch.int64, device=dev)
-        return self.forward(plan, ids_dev, last)
+        both = torch.tensor(ids + plan_last_rows(plan), dtype=torch.int64, pin_memory=True)
+        both = both.to(self.w.embedding.device, non_blocking=True)
+        return self.forward(plan, both[:len(ids)], both[len(ids):])
 
     def forward(self, plan: StepPlan, ids: torch.Tensor, last_rows: torch.Tensor) -> torch.Tensor:
         cfg, w = self.cfg, self.w

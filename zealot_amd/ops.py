@@ -15,28 +15,38 @@ import torch
 
 from . import _lib
 
-_FP8_DTYPES = tuple(d for d in (getattr(torch, "float8_e4m3fn", None), torch.uint8) if d is not None)
+_ZK_DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.uint8: _lib.FP8_E4M3}
+if hasattr(torch, "float8_e4m3fn"):
+    _ZK_DTYPES[torch.float8_e4m3fn] = _lib.FP8_E4M3
 
 
 def zk_dtype(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return _lib.F32
-    if t.dtype == torch.bfloat16:
-        return _lib.BF16
-    if t.dtype in _FP8_DTYPES:
-        return _lib.FP8_E4M3
-    raise TypeError(f"unsupported dtype {t.dtype}")
+    code = _ZK_DTYPES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}")
+    return code
 
 
-def _stream(stream=None) -> ctypes.c_void_p:
-    s = torch.cuda.current_stream() if stream is None else stream
-    return ctypes.c_void_p(s.cuda_stream)
+# The current stream's handle without the torch.cuda.Stream object around it:
+# 0.2 us against 2.9, in calls whose launch takes 3.7 (a one-token append: 9.9 us
+# of host time before, 5.5 with this and the checks below).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def _stream(stream=None) -> int:
+    """The address of `stream`, by default torch's current stream."""
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or _get_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_get_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None, contiguous=True) -> int:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be on a GPU (got {t.device})")
     if contiguous and not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
@@ -50,9 +60,10 @@ def _opt(t, name, dtype=None):
 
 
 def _pool_shape(k_pool: torch.Tensor, v_pool: torch.Tensor):
-    if k_pool.dim() != 4 or k_pool.shape != v_pool.shape or k_pool.dtype != v_pool.dtype:
+    shape = k_pool.shape
+    if len(shape) != 4 or shape != v_pool.shape or k_pool.dtype != v_pool.dtype:
         raise ValueError("k_pool/v_pool must be equal 4-D tensors [num_blocks, Hkv, block_size, D]")
-    return tuple(int(x) for x in k_pool.shape)
+    return shape
 
 
 def append(k_pool, v_pool, k, v, slot_mapping, k_scales=None, v_scales=None, token_row=None,
@@ -136,9 +147,8 @@ def paged_decode(q, k_pool, v_pool, block_tables, seq_lens, scale=None, mapping=
         out = torch.empty_like(q)
     elif out.shape != q.shape or out.dtype != q.dtype:
         raise ValueError("out must match q")
-    need = decode_workspace_bytes(n, h, d, mb, bs)
-    if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    if workspace is None:  # (one that is given is checked by the call)
+        workspace = torch.empty(decode_workspace_bytes(n, h, d, mb, bs), dtype=torch.uint8, device=q.device)
     _lib.check(_lib.lib().zk_paged_decode(
         _dev(q, "q"), zk_dtype(q), _dev(k_pool, "k_pool"), _dev(v_pool, "v_pool"),
         zk_dtype(k_pool), _dev(out, "out"), _dev(block_tables, "block_tables", torch.int32),
@@ -172,9 +182,8 @@ def paged_prefill(q, k_pool, v_pool, block_tables, cu_seqlens_q, start_pos, caus
         out = torch.empty_like(q)
     elif out.shape != q.shape or out.dtype != q.dtype:
         raise ValueError("out must match q")
-    need = prefill_workspace_bytes(n, t, h, hkv)
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        workspace = torch.empty(prefill_workspace_bytes(n, t, h, hkv), dtype=torch.uint8, device=q.device)
     _lib.check(_lib.lib().zk_paged_prefill(
         _dev(q, "q"), zk_dtype(q), _dev(k_pool, "k_pool"), _dev(v_pool, "v_pool"), zk_dtype(k_pool),
         _dev(out, "out"), _dev(block_tables, "block_tables", torch.int32),
