@@ -1256,6 +1256,9 @@ int decode_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState 
     const float *dvs = fp8 ? dks + (size_t)n * H : nullptr;
     const int32_t *dsh = (const int32_t *)(d + len_bytes + sc_bytes);
     zk::PrefixGroups pg{dsh + o_pb, dsh + o_mem, dsh + o_pages, nsg, sp.total_pages};
+    for (int32_t x : sp.sg_pages) pg.max_pages = std::max(pg.max_pages, (int)x);
+    for (int i = 0; nsg && i < n; ++i)
+        pg.max_rest = std::max(pg.max_rest, (int)((lens[i] + c->block_size - 1) / c->block_size) - sp.seq_pb[i]);
     c->last_sg = nsg;
     c->last_sg_pages = sp.total_pages;
     const int32_t *drows = q_rows ? (const int32_t *)(d + len_bytes + sc_bytes + share_bytes) : nullptr;

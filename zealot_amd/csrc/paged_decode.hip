@@ -133,6 +133,7 @@ struct Params {
     const int32_t *sg_members;
     const int32_t *sg_pages;
     int num_sg, shared_part_pages;
+    int shared_parts;  // planless: partitions of the longest shared prefix
     int num_seqs, num_heads, num_kv_heads, head_dim, block_size, max_blocks, part_pages, max_parts;
     int64_t num_blocks;
     float scale_log2;  // softmax scale * log2(e)
@@ -433,7 +434,9 @@ struct LdsVec<4> { typedef uint32_t T; };
 // behind 0..600 tokens, 32 / 8 heads of 128: 57 us as 150 one-row decodes, 31
 // here, and its tables no longer displace the decode half's (four uploads of a
 // step gone): the step of it and 12 decodes 113 -> 60 us.
-template <int KV, int D, int G, bool DIRECT, bool ROWS = false>
+// SHARED (with DIRECT): the first num_sg * shared_parts workgroups of a kv-head
+// are the shared-prefix partitions, the others the sequences' own.
+template <int KV, int D, int G, bool DIRECT, bool ROWS = false, bool SHARED = false>
 __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     constexpr int BS = 16;
     constexpr int BIDS = DIRECT && !ROWS ? kDirectPages : kMaxItemPages;
@@ -869,6 +872,46 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     };
     const u32x4 no_row = {0u, 0u, 0u, 0u};
 
+    // shared-prefix partition `part` of subgroup sg (np pages of member 0's table)
+    auto shared_part = [&](int sg, int kvh, int part, int n0, int np, int4 d1) {
+        // shared-prefix partition of subgroup sg: up to 32 rows, member-major
+        const int page0 = part * p.shared_part_pages;
+        // members (batch indices) of the subgroup, by scalar loads; lane
+        // (grp, col) serves row r = 16 t + col, member r / G
+        constexpr int NM = kSgStride / G;
+        const cint_t cmem = (cint_t)(p.sg_members + (size_t)sg * kSgStride);
+        int mem_s[NM];
+#pragma unroll
+        for (int j = 0; j < NM; ++j) mem_s[j] = cmem[j];
+        qfrag_t qf[2][KK];
+        int nm[2];  // member of this lane's row in tile t, or -1
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int r = 16 * t + col;
+            int v = mem_s[0];
+#pragma unroll
+            for (int j = 1; j < NM; ++j) v = r / G == j ? mem_s[j] : v;
+            nm[t] = v;
+            if (nm[t] >= 0) load_q(q_row(nm[t]), qhead_of(p, kvh, r % G, G), qf[t]);
+            else
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) qf[t][kk] = qzero;
+        }
+        f32x4 o[DT][2];
+        float m[2], l[2];
+        const int all[2] = {0x7fffffff, 0x7fffffff};
+        attend.template operator()<2>(qf, p.bt + (size_t)n0 * p.max_blocks + page0, d1, page0, np, 0x7fffffff, all,
+                                      kvh, p.scale_log2, o, m, l, -1, no_row, 0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int r = 16 * t + col;
+            if (nm[t] >= 0) {
+                const size_t slot = ((size_t)nm[t] * H + qhead_of(p, kvh, r % G, G)) * p.max_parts + part;
+                store_partial(slot, o, t, 1.0f, m[t], l[t]);
+            }
+        }
+    };
+
     // a sequence's own partition: rows 0..G-1 are its heads of kv-head kvh
     // (ns shared and nparts own partitions in all; cut: the partition's pages
     // end at an invalid table entry)
@@ -1002,7 +1045,45 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         }
         return;
     }
-    if constexpr (DIRECT && !ROWS) {
+    if constexpr (SHARED) {
+        const int kvh = blockIdx.x, items = p.num_sg * p.shared_parts;
+        int y = blockIdx.y;
+        const bool sh = y < items;
+        int n, part, page0, pages, len = 0, ns = 0, nparts = 0, sg = 0;  // pages of the partition
+        if (sh) {
+            sg = y / p.shared_parts;
+            part = y % p.shared_parts;
+            n = ((cint_t)p.sg_members)[(size_t)sg * kSgStride];
+            page0 = part * p.shared_part_pages;
+            pages = min(p.shared_part_pages, ((cint_t)p.sg_pages)[sg] - page0);
+            if (pages <= 0) return;
+        } else {
+            y -= items;
+            const int own = p.max_parts - p.shared_parts;
+            n = y / own;
+            part = y % own;
+            len = min(max(((cint_t)p.seq_lens)[n], 0), p.max_blocks * BS);
+            const int pb = ((cint_t)p.seq_pb)[n], rest = (len + BS - 1) / BS - pb;
+            ns = pb > 0 ? (pb + p.shared_part_pages - 1) / p.shared_part_pages : 0;
+            nparts = rest > 0 ? (rest + p.part_pages - 1) / p.part_pages : 0;
+            if (part >= (ns == 0 ? max(1, nparts) : nparts)) return;
+            page0 = pb + part * p.part_pages;
+            pages = max(0, min(p.part_pages, rest - part * p.part_pages));
+        }
+        // (the cache's tables: valid up to every length; an id outside the pool
+        // still ends the walk)
+        const int e = pages > 0 ? p.bt[(size_t)n * p.max_blocks + page0 + min(lane, pages - 1)] : 0;
+        const uint64_t bad = __builtin_amdgcn_ballot_w64(lane < pages && (e < 0 || (int64_t)e >= p.num_blocks));
+        const int np = bad ? (int)__builtin_ctzll(bad) : pages;
+        bids[lane] = e;
+        wait_lgkmcnt0();
+        const int4 first = make_int4(__builtin_amdgcn_readlane(e, 0), __builtin_amdgcn_readlane(e, 1),
+                                     __builtin_amdgcn_readlane(e, 2), __builtin_amdgcn_readlane(e, 3));
+        if (sh) shared_part(sg, kvh, part, n, np, first);
+        else own_part(n, kvh, part, page0, np, len, ns, nparts, first, bad != 0);
+        return;
+    }
+    if constexpr (DIRECT && !ROWS && !SHARED) {
         const int kvh = blockIdx.x, part = blockIdx.y, n = blockIdx.z;
         const int page0 = part * p.part_pages;
         const int32_t *row = p.bt + (size_t)n * p.max_blocks;
@@ -1032,43 +1113,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         bool own = true;
         if constexpr (KV == ZK_BF16) own = d0.x >= 0;
         if (!own) {
-            // shared-prefix partition of subgroup sg: up to 32 rows, member-major
-            const int sg = -1 - d0.x, part = d0.y, n0 = d0.z, np = d0.w;
-            const int page0 = part * p.shared_part_pages;
-            // members (batch indices) of the subgroup, by scalar loads; lane
-            // (grp, col) serves row r = 16 t + col, member r / G
-            constexpr int NM = kSgStride / G;
-            const cint_t cmem = (cint_t)(p.sg_members + (size_t)sg * kSgStride);
-            int mem_s[NM];
-#pragma unroll
-            for (int j = 0; j < NM; ++j) mem_s[j] = cmem[j];
-            qfrag_t qf[2][KK];
-            int nm[2];  // member of this lane's row in tile t, or -1
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int r = 16 * t + col;
-                int v = mem_s[0];
-#pragma unroll
-                for (int j = 1; j < NM; ++j) v = r / G == j ? mem_s[j] : v;
-                nm[t] = v;
-                if (nm[t] >= 0) load_q(q_row(nm[t]), qhead_of(p, kvh, r % G, G), qf[t]);
-                else
-#pragma unroll
-                    for (int kk = 0; kk < KK; ++kk) qf[t][kk] = qzero;
-            }
-            f32x4 o[DT][2];
-            float m[2], l[2];
-            const int all[2] = {0x7fffffff, 0x7fffffff};
-            attend.template operator()<2>(qf, p.bt + (size_t)n0 * p.max_blocks + page0, d1, page0, np, 0x7fffffff, all,
-                                          kvh, p.scale_log2, o, m, l, -1, no_row, 0);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int r = 16 * t + col;
-                if (nm[t] >= 0) {
-                    const size_t slot = ((size_t)nm[t] * H + qhead_of(p, kvh, r % G, G)) * p.max_parts + part;
-                    store_partial(slot, o, t, 1.0f, m[t], l[t]);
-                }
-            }
+            shared_part(-1 - d0.x, kvh, d0.y, d0.z, d0.w, d1);
         } else {
             const int n = d0.x, part = d0.y, page0 = d0.z, np = d0.w;
             const int len = ((cint_t)p.eff_len)[n];  // walk already cut at the first invalid entry
@@ -1561,7 +1606,13 @@ int persistent_grid() {
 
 template <int KV, int D, int G>
 void launch_mfma_k(const Params &p, hipStream_t s) {
-    if (p.num_waves > 0)
+    if (p.num_waves == 0 && p.num_sg > 0) {
+        if constexpr (KV == ZK_BF16) {
+            const int own = p.max_parts - p.shared_parts;
+            const dim3 grid(p.num_kv_heads, p.num_sg * p.shared_parts + p.num_seqs * own);
+            decode_mfma_kernel<KV, D, G, true, false, true><<<grid, kWave, 0, s>>>(p);
+        }
+    } else if (p.num_waves > 0)
         decode_mfma_kernel<KV, D, G, false><<<p.num_waves, kWave, 0, s>>>(p);
     else
         decode_mfma_kernel<KV, D, G, true><<<dim3(p.num_kv_heads, p.max_parts, p.num_seqs), kWave, 0, s>>>(p);
@@ -1662,6 +1713,14 @@ int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves)
 // than 8 pages do not pay for the reduce; the count is rounded to the nearest
 // so that a table a little over P stays one partition (no reduce at all).
 constexpr double kDirectBytes = 3e9;
+// Shared prefixes without a plan: about this many shared items over all
+// kv-heads (each streams its pages for up to 32 rows, beside the sequences' own
+// one- and two-page items, all resident at once), of at least 10 pages.  Against
+// the planned launch (eight queues, 32-page items), four layers of a step, us: 16
+// x 8 forks of 2050 tokens 152 / 139, 12 x 8 of 3900 187 / 172, 5 x 11 of 2420 117 /
+// 107, 8 x 2 of 700 76 / 62, 1 x 2 of 400 70 / 45; 256, 512, 640 and 1024 items 171,
+// 146, 147 and 161 on the first.
+constexpr long kSharedItems = 384, kSharedMinPages = 10;
 int direct_parts(double units, double page_bytes, int max_blocks) {
     const double bytes = units * page_bytes;
     if (bytes > kDirectBytes) return 0;
@@ -1722,6 +1781,7 @@ int check_decode_args(zk_dtype q_dtype, zk_dtype kv_dtype, int num_seqs, int num
 // needs (arguments already checked).
 struct DecodeShape {
     bool use_mfma, shared, direct;
+    int shared_parts;
     int part_pages, shared_pages, max_parts, waves;
     WsLayout w;
 };
@@ -1747,6 +1807,26 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
                            : max_parts_for(max_blocks_per_seq, d.part_pages);
     d.w = ws_layout(num_seqs, num_heads, head_dim, d.max_parts);
     d.direct = false;
+    d.shared_parts = 0;
+    if (d.use_mfma && d.shared && max_waves == 0 && !part_pages_env() && pg->max_pages > 0) {
+        // shared prefixes without a plan: see kSharedItems
+        const double page_bytes = 2.0 * block_size * head_dim * elt_size(kv_dtype);
+        const double own_units = (double)num_seqs * std::max(1, pg->max_rest) * num_kv_heads;
+        const int own = direct_parts(own_units, page_bytes, std::max(1, pg->max_rest));
+        const int sp = (int)std::min<long>(kDirectPages, std::max<long>(kSharedMinPages, (pg->total_shared_pages * num_kv_heads + kSharedItems - 1) / kSharedItems));
+        const int parts = (pg->max_pages + sp - 1) / sp;
+        const WsLayout w = ws_layout(num_seqs, num_heads, head_dim, parts + own);
+        if (own > 0 && (own_units + (double)pg->total_shared_pages * num_kv_heads) * page_bytes <= kDirectBytes &&
+            (long)pg->num_sg * parts + (long)num_seqs * own <= 65535 && w.total <= workspace_bytes) {
+            d.direct = true;
+            d.waves = 0;
+            d.shared_parts = parts;
+            d.shared_pages = sp;
+            d.part_pages = (std::max(1, pg->max_rest) + own - 1) / own;
+            d.max_parts = parts + own;
+            d.w = w;
+        }
+    }
     if (d.use_mfma && !d.shared && max_waves == 0 && !part_pages_env()) {
         const int parts = direct_parts((double)num_seqs * max_blocks_per_seq * num_kv_heads,
                                        2.0 * block_size * head_dim * elt_size(kv_dtype), max_blocks_per_seq);
@@ -1837,6 +1917,7 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
     p.sg_pages = shared ? pg->sg_pages : nullptr;
     p.num_sg = shared ? pg->num_sg : 0;
     p.shared_part_pages = shared ? shared_pages : 1;
+    p.shared_parts = ds.shared_parts;
     p.scale_log2 = scale * kLog2e;
     p.grouped = mapping == ZK_GQA_GROUPED ? 1 : 0;
     p.q_f32 = q_dtype == ZK_F32 ? 1 : 0;

@@ -90,6 +90,8 @@ struct PrefixGroups {
     const int32_t *sg_pages;
     int num_sg;
     long total_shared_pages;
+    int max_pages = 0;  // most shared pages of a subgroup (0: not known)
+    int max_rest = 0;   // most pages of a sequence after its shared ones
 };
 // zk_paged_decode with optional shared prefixes (pg may be null), an
 // optional device map from sequence to q / out row (q_rows may be null), the
