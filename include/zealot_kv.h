@@ -138,6 +138,13 @@ int zk_append(void *k_pool, void *v_pool, zk_dtype cache_dtype, const void *k, c
 int zk_fp8_scales(const void *x, zk_dtype src_dtype, const int64_t *cu_seqlens, int num_seqs,
                   int num_kv_heads, int head_dim, float *scales, void *stream);
 
+/* The same with every sequence's tokens cut into `parts` parts that workgroups
+ * of their own go through (long prompts in small batches): maxima is device
+ * scratch of parts * num_seqs * num_kv_heads floats (unused for parts = 1).
+ * Same values. */
+int zk_fp8_scales_parts(const void *x, zk_dtype src_dtype, const int64_t *cu_seqlens, int num_seqs, int num_kv_heads,
+                        int head_dim, float *scales, float *maxima, int parts, void *stream);
+
 /* Block-table gather: pages -> contiguous token-major rows.  For sequence n,
  * its first ctx_lens[n] tokens (walk stops at a negative table entry, as
  * paged_attention.cu:63-83) land in rows [out_offsets[n], out_offsets[n] +

@@ -89,6 +89,7 @@ SIGNATURES = {
     "zk_bm_check": (_I, [_P, BlockHandleC]),
     "zk_append": (_I, [_P, _P, _I, _P, _P, _I, _P, _I64, _I, _I, _I, _I64, _P, _P, _P, _P]),
     "zk_fp8_scales": (_I, [_P, _I, _P, _I, _I, _I, _P, _P]),
+    "zk_fp8_scales_parts": (_I, [_P, _I, _P, _I, _I, _I, _P, _P, _I, _P]),
     "zk_gather": (_I, [_P, _P, _I, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I64, _P]),
     "zk_copy_blocks": (_I, [_P, _I, _I64, _I64, _P, _P, _I64, _P]),
     "zk_paged_decode_workspace_size": (_SZ, [_I, _I, _I, _I, _I]),

@@ -267,23 +267,28 @@ __device__ __forceinline__ float amax16(uint4 w) {
     return m;
 }
 
-// One workgroup per (sequence, kv head), a 1024-thread one since the sequences
-// of a prompt batch are few: the head's rows are read as one line of 16-byte
-// chunks, consecutive lanes consecutive chunks of a row, eight loads a thread in
-// flight.  Bound by what one CU can have in flight: 12 prompts of 60..2000
-// tokens, 8 heads of 128 bf16 (28 MB) 15 us (37 us with a whole row a
-// thread, whose loads touch 64 lines each).  Rows that are not 16-byte chunks
-// go element by element.
-constexpr int kScaleThreads = 1024;
+// One workgroup per (sequence, kv head, part of its tokens): the head's rows are
+// read as one line of 16-byte chunks, consecutive lanes consecutive chunks of a
+// row, eight loads a thread in flight.  12 prompts of 60..2000 tokens, 8 heads of
+// 128 bf16 (28 MB): 37 us with a whole row a thread (its loads touch 64 lines
+// each), 15 with one part, bound by what the longest prompt's CU can have in
+// flight, 9 with parts and the merge of their maxima (fp8_scales_merge_kernel).  Rows
+// that are not 16-byte chunks go element by element.
+constexpr int kScaleThreads = 512;
 template <int SRC, bool VEC>
 __global__ void __launch_bounds__(kScaleThreads)
 fp8_scales_kernel(const void *__restrict__ x, const int64_t *__restrict__ cu, uint32_t hkv, uint32_t head_dim,
-                  float *__restrict__ scales) {
+                  float *__restrict__ scales, float *__restrict__ maxima) {
     constexpr int U = 8;
     constexpr uint32_t ES = SRC == ZK_F32 ? 4 : 2;
     __shared__ float red[kScaleThreads / 64];
     const uint32_t n = blockIdx.x, h = blockIdx.y;
-    const int64_t t0 = cu[n], t1 = cu[n + 1];
+    int64_t t0 = cu[n], t1 = cu[n + 1];
+    if (gridDim.z > 1) {  // this part's tokens
+        const int64_t per = (t1 - t0 + gridDim.z - 1) / gridDim.z;
+        t0 += (int64_t)blockIdx.z * per;
+        t1 = t1 < t0 + per ? t1 : t0 + per;
+    }
     float amax = 0.0f;
     if (t1 > t0) {
         const uint64_t per_row = VEC ? head_dim * ES / 16 : head_dim, total = (uint64_t)(t1 - t0) * per_row;
@@ -319,8 +324,19 @@ fp8_scales_kernel(const void *__restrict__ x, const int64_t *__restrict__ cu, ui
     if (threadIdx.x == 0) {
         float m = red[0];
         for (int i = 1; i < kScaleThreads / 64; ++i) m = fmaxf(m, red[i]);
-        scales[(size_t)n * hkv + h] = m > 0.0f ? m / 448.0f : 1.0f;
+        if (gridDim.z > 1) maxima[((size_t)blockIdx.z * gridDim.x + n) * hkv + h] = m;
+        else scales[(size_t)n * hkv + h] = m > 0.0f ? m / 448.0f : 1.0f;
     }
+}
+
+// scales of `count` (sequence, head)s from the maxima of their parts.
+__global__ void __launch_bounds__(kThreads)
+fp8_scales_merge_kernel(const float *__restrict__ maxima, int parts, int count, float *__restrict__ scales) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= count) return;
+    float m = 0.0f;
+    for (int c = 0; c < parts; ++c) m = fmaxf(m, maxima[(size_t)c * count + i]);
+    scales[i] = m > 0.0f ? m / 448.0f : 1.0f;
 }
 
 // ------------------------------------------------------------------ gather
@@ -674,20 +690,35 @@ extern "C" {
 
 int zk_fp8_scales(const void *x, zk_dtype src_dtype, const int64_t *cu_seqlens, int num_seqs,
                   int num_kv_heads, int head_dim, float *scales, void *stream) {
+    return zk_fp8_scales_parts(x, src_dtype, cu_seqlens, num_seqs, num_kv_heads, head_dim, scales, nullptr, 1, stream);
+}
+
+int zk_fp8_scales_parts(const void *x, zk_dtype src_dtype, const int64_t *cu_seqlens, int num_seqs, int num_kv_heads,
+                        int head_dim, float *scales, float *maxima, int parts, void *stream) {
     if (src_dtype != ZK_F32 && src_dtype != ZK_BF16)
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_fp8_scales: unsupported dtype");
-    if (num_seqs < 0 || num_kv_heads <= 0 || head_dim <= 0)
+    if (num_seqs < 0 || num_kv_heads <= 0 || head_dim <= 0 || parts < 1 || parts > 65535)
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_fp8_scales: bad shape");
     if (num_seqs == 0) return ZK_OK;
-    if (!x || !cu_seqlens || !scales)
+    if (!x || !cu_seqlens || !scales || (parts > 1 && !maxima))
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_fp8_scales: NULL pointer");
-    dim3 grid(num_seqs, num_kv_heads);
-    KernelTimer timer("fp8_scales", (hipStream_t)stream);
     const bool vec = ((size_t)head_dim * elt_size(src_dtype)) % 16 == 0 && ((uintptr_t)x & 15u) == 0;
     auto kernel = src_dtype == ZK_F32 ? (vec ? fp8_scales_kernel<ZK_F32, true> : fp8_scales_kernel<ZK_F32, false>)
                                       : (vec ? fp8_scales_kernel<ZK_BF16, true> : fp8_scales_kernel<ZK_BF16, false>);
-    kernel<<<grid, kScaleThreads, 0, (hipStream_t)stream>>>(x, cu_seqlens, num_kv_heads, head_dim, scales);
-    return check_launch("zk_fp8_scales");
+    const hipStream_t s = (hipStream_t)stream;
+    {
+        KernelTimer timer("fp8_scales", s);
+        kernel<<<dim3(num_seqs, num_kv_heads, parts), kScaleThreads, 0, s>>>(x, cu_seqlens, num_kv_heads, head_dim, scales,
+                                                                             maxima);
+    }
+    if (int rc = check_launch("zk_fp8_scales")) return rc;
+    if (parts == 1) return ZK_OK;
+    const int64_t count = (int64_t)num_seqs * num_kv_heads;
+    if (count > 0x7fffffff)
+        return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_fp8_scales: bad shape");
+    KernelTimer timer("fp8_scales_merge", s);
+    fp8_scales_merge_kernel<<<(uint32_t)((count + kThreads - 1) / kThreads), kThreads, 0, s>>>(maxima, parts, (int)count, scales);
+    return check_launch("zk_fp8_scales merge");
 }
 
 int zk_gather(const void *k_pool, const void *v_pool, zk_dtype dtype, const int32_t *block_tables,

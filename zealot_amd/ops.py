@@ -85,10 +85,16 @@ def append(k_pool, v_pool, k, v, slot_mapping, k_scales=None, v_scales=None, tok
 def fp8_scales(x, cu_seqlens, stream=None) -> torch.Tensor:
     """Per-(sequence, kv_head) scales amax/448 over x[cu[n]:cu[n+1]] ([T, Hkv, D])."""
     n = cu_seqlens.shape[0] - 1
-    out = torch.empty((n, x.shape[1]), dtype=torch.float32, device=x.device)
-    _lib.check(_lib.lib().zk_fp8_scales(
-        _dev(x, "x"), zk_dtype(x), _dev(cu_seqlens, "cu_seqlens", torch.int64), n, x.shape[1],
-        x.shape[2], out.data_ptr(), _stream(stream)))
+    tokens, hkv, d = x.shape
+    out = torch.empty((n, hkv), dtype=torch.float32, device=x.device)
+    # parts of at least 64 tokens on average, up to two workgroups a CU: below,
+    # the second launch costs more than the parts give.  (Not on a stream of the
+    # caller's choice: the scratch belongs to the current one.)
+    parts = min(512 // max(1, n * hkv), tokens // (64 * max(1, n))) if stream is None else 1
+    scratch = torch.empty(parts * n * hkv, dtype=torch.float32, device=x.device) if parts > 1 else None
+    _lib.check(_lib.lib().zk_fp8_scales_parts(
+        _dev(x, "x"), zk_dtype(x), _dev(cu_seqlens, "cu_seqlens", torch.int64), n, hkv, d, out.data_ptr(),
+        scratch.data_ptr() if parts > 1 else None, max(1, parts), _stream(stream)))
     return out
 
 
