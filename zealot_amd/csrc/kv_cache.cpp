@@ -1503,8 +1503,19 @@ int zk_cache_attention_batch(zk_kv_cache *c, size_t layer, const char *const *id
         if (!dec.empty()) {
             if (int rc = ensure_side_stream(c)) return rc;
             ps = c->side;
-            pre_groups = c->cus;
-            dec_waves = 2 * c->cus;
+            // a decode of up to kSmallDecode bytes of K and V is over before the
+            // shares would matter: both kernels then take what is free (60 decodes
+            // of 50..800 tokens and 3 chunks of 500: 148 us in shares, 113; 8 of
+            // 50..6000 and 3 of 512: 84 and 66; from 200 MB on shares win again,
+            // 100 of 50..1000 and 3 of 300: 123 and 139)
+            constexpr double kSmallDecode = 128e6;
+            const double token_bytes = 2.0 * (double)(c->num_kv_heads * c->head_dim) * zk::elt_size(c->dtype);
+            double dec_bytes = 0;
+            for (const SeqState *d : dec) dec_bytes += token_bytes * (double)d->layer_len[layer];
+            if (dec_bytes > kSmallDecode) {
+                pre_groups = c->cus;
+                dec_waves = 2 * c->cus;
+            }
         }
         int64_t chunk_rows = 0;  // sizes the launch: the decode rows are not its
         for (int32_t l : pre_len) chunk_rows += l;
