@@ -1782,6 +1782,7 @@ int check_decode_args(zk_dtype q_dtype, zk_dtype kv_dtype, int num_seqs, int num
 struct DecodeShape {
     bool use_mfma, shared, direct;
     int shared_parts;
+    size_t need;  // workspace a caller must give: the planned launch's, also where the planless one takes less
     int part_pages, shared_pages, max_parts, waves;
     WsLayout w;
 };
@@ -1806,8 +1807,14 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
     d.max_parts = d.shared ? max_parts_for(max_blocks_per_seq, min_part_pages(head_dim, block_size)) + 1
                            : max_parts_for(max_blocks_per_seq, d.part_pages);
     d.w = ws_layout(num_seqs, num_heads, head_dim, d.max_parts);
+    d.need = d.w.total;
+    if (d.use_mfma && kv_dtype == ZK_F32)  // (as the generic kernel cuts the contexts)
+        d.need = std::max(d.need, ws_layout(num_seqs, num_heads, head_dim,
+                                            max_parts_for(max_blocks_per_seq, part_pages_for(ZK_F32, head_dim, block_size)))
+                                      .total);
     d.direct = false;
     d.shared_parts = 0;
+    if (workspace_bytes < d.need) return d;  // refused
     if (d.use_mfma && d.shared && max_waves == 0 && !part_pages_env() && pg->max_pages > 0) {
         // shared prefixes without a plan: see kSharedItems
         const double page_bytes = 2.0 * block_size * head_dim * elt_size(kv_dtype);
@@ -1839,6 +1846,7 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
             d.w = w;
         }
     }
+    d.need = std::max(d.need, d.w.total);
     return d;
 }
 
@@ -1878,10 +1886,10 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
                          "16-byte aligned rows");
     const int part_pages = ds.part_pages, shared_pages = ds.shared_pages, max_parts = ds.max_parts;
     const WsLayout &w = ds.w;
-    if (workspace_bytes < w.total || ((uintptr_t)workspace & 255u))
+    if (workspace_bytes < ds.need || ((uintptr_t)workspace & 255u))
         return set_error(ZK_ERR_INVALID_ARGUMENT,
                          "Internal error: zk_paged_decode: workspace too small or not 256-B aligned (need " +
-                             std::to_string(w.total) + " bytes)");
+                             std::to_string(ds.need) + " bytes)");
 
     Params p{};
     p.q = q;
@@ -2114,7 +2122,7 @@ int zk_paged_decode_noalloc(const void *q, zk_dtype q_dtype, const void *k_pool,
         decode_shape(kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, nullptr,
                      (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool | (uintptr_t)out) & 15u) == 0,
                      (size_t)ZK_DECODE_SCRATCH_BYTES)
-            .w.total;
+            .need;
     if (need > (size_t)ZK_DECODE_SCRATCH_BYTES)
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: zk_paged_decode_noalloc: the call needs " +
                                                       std::to_string(need) + " bytes of scratch, the maximum is " +
