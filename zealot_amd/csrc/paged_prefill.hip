@@ -37,8 +37,8 @@
 // (one prompt's chunk behind a long context) split each over its keys;
 // prefill_reduce_kernel merges the splits.  A 389-token chunk behind 7680
 // tokens, 32 / 8 heads of 128 bf16: 167 us planned (104 workgroups on 256
-// CUs), 82 us in four splits (75 attention, bound by the CUs that hold two of
-// the 416 workgroups, 8 merge); a 20-token chunk behind 100: 17 and 15 us, host
+// CUs), 75 us in four splits (bound by the CUs that hold two of
+// the 416 workgroups, and 8 of merge); a 20-token chunk behind 100: 17 and 15 us, host
 // time the most of it.
 #include <hip/hip_runtime.h>
 
