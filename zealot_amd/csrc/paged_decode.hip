@@ -1800,6 +1800,8 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
     if (max_waves > 0 && max_waves < d.waves) d.waves = max_waves;
     d.part_pages = d.use_mfma ? mfma_part_pages(num_seqs, num_kv_heads, max_blocks_per_seq, d.waves)
                               : part_pages_for(ZK_F32, head_dim, block_size);
+    // (no smaller than the generic kernel's: one workspace serves both)
+    if (kv_dtype == ZK_F32) d.part_pages = std::max(d.part_pages, part_pages_for(ZK_F32, head_dim, block_size));
     d.shared = pg && pg->num_sg > 0 &&
                paged_decode_shares_prefixes(kv_dtype, head_dim, block_size, num_heads, num_kv_heads);
     d.shared_pages = d.shared ? shared_part_pages_for(pg->total_shared_pages, num_kv_heads, d.waves) : 0;
@@ -1808,7 +1810,7 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
                            : max_parts_for(max_blocks_per_seq, d.part_pages);
     d.w = ws_layout(num_seqs, num_heads, head_dim, d.max_parts);
     d.need = d.w.total;
-    if (d.use_mfma && kv_dtype == ZK_F32)  // (as the generic kernel cuts the contexts)
+    if (d.use_mfma && kv_dtype == ZK_F32)  // (as the generic kernel, which takes the unaligned calls, needs)
         d.need = std::max(d.need, ws_layout(num_seqs, num_heads, head_dim,
                                             max_parts_for(max_blocks_per_seq, part_pages_for(ZK_F32, head_dim, block_size)))
                                       .total);
