@@ -4,6 +4,7 @@ K / V: chunk lengths around a group, contexts of one and of several partitions,
 chunks beside decodes, both mappings, head counts and sizes, bf16 queries,
 strided and unaligned queries (the latter take the per-row decodes).  Tolerance
 1e-5 absolute (f32), 2e-2 for bf16 outputs."""
+import ctypes
 import math
 
 import pytest
@@ -63,3 +64,31 @@ def test_chunks_match_float64(H, Hkv, D, mapping, qdt, layout):
         want = _ref(q[row:row + t], k, v, H, Hkv, mapping, b)
         assert (got[row:row + t] - want).abs().max() <= (1e-5 if qdt == torch.float32 else 2e-2)
         row += t
+
+
+def test_chunk_only_steps_refuse_what_decodes_refuse():
+    """A step of chunks alone, as one with a decode beside them: a query type that
+    is not f32 or bf16, an unknown head mapping."""
+    from zealot_amd import BlockManager, KVCache, ZealotError, _lib
+    from zealot_amd.kv_cache import SeqBatch
+    H, Hkv, D, t = 8, 2, 128, 20
+    bm = BlockManager(8, 16)
+    cache = KVCache(8, 16, 1, Hkv, D, dtype=torch.float32, max_seqs=2, max_blocks_per_seq=4)
+    cache.register_seq("s", 4)
+    for _ in range(2):
+        cache.alloc_block("s", bm)
+    kv = torch.zeros((t, Hkv, D), device="cuda")
+    cache.write_batch(0, ["s"], [t], kv, kv)
+    out = torch.full((t, H, D), 7.0, device="cuda")
+    q = torch.zeros((t, H, D), device="cuda")
+    for dtype in (torch.uint8, torch.float8_e4m3fn):
+        with pytest.raises(ZealotError, match="q dtype"):
+            cache.attention_batch(0, ["s"], [t], torch.zeros((t, H, D), dtype=torch.uint8, device="cuda").view(dtype))
+    b, n = SeqBatch(["s"]), (ctypes.c_int32 * 1)(t)
+    for qdt, mapping, what in ((_lib.FP8_E4M3, _lib.GQA_GROUPED, "q dtype"), (7, _lib.GQA_GROUPED, "q dtype"), (_lib.F32, 7, "mapping")):
+        rc = _lib.lib().zk_cache_attention_batch(cache._h, 0, b.arr, ctypes.addressof(n), 1, q.data_ptr(), qdt, 0, out.data_ptr(), H,
+                                                 0.1, mapping)
+        with pytest.raises(ZealotError, match=what):
+            _lib.check(rc)
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())  # nothing was launched

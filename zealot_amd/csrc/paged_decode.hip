@@ -2044,7 +2044,12 @@ int zk::paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const vo
                    const int32_t *block_tables, const int4 *row_groups, int groups, int num_heads, int num_kv_heads,
                    int head_dim, int max_blocks_per_seq, int64_t num_blocks, float scale, zk_gqa_mapping mapping,
                    void *workspace, size_t workspace_bytes, void *stream, int64_t q_stride) {
-    if (groups <= 0) return ZK_OK;
+    if (int rc = check_decode_args(q_dtype, ZK_F32, groups, num_heads, num_kv_heads, head_dim, 16, max_blocks_per_seq,
+                                   num_blocks, mapping))
+        return rc;
+    if (groups == 0) return ZK_OK;
+    if (!q || !k_pool || !v_pool || !out || !block_tables || !row_groups || !workspace)
+        return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged rows: NULL pointer");
     const WsLayout w = rows_layout(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq);
     if (groups > 65535 || workspace_bytes < w.total || ((uintptr_t)workspace & 255u))
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged rows: too many groups or workspace too small");
