@@ -92,3 +92,36 @@ def test_chunk_only_steps_refuse_what_decodes_refuse():
             _lib.check(rc)
     torch.cuda.synchronize()
     assert bool((out == 7.0).all())  # nothing was launched
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (4, 4, 64), (16, 2, 128)])
+@pytest.mark.parametrize("before,t", [(0, 40), (13, 70), (600, 33)])
+def test_rows_do_not_see_later_tokens_infinities(H, Hkv, D, before, t):
+    """Infinities and NaN in K and V of a token reach the rows from that token
+    on and no earlier one, also inside a row group and a page; every row against
+    float64 attention of its own keys alone."""
+    from zealot_amd import BlockManager, KVCache
+    bm = BlockManager(60, 16)
+    cache = KVCache(60, 16, 1, Hkv, D, dtype=torch.float32, max_seqs=1, max_blocks_per_seq=50)
+    g = torch.Generator().manual_seed(H + before)
+    n = before + t
+    k, v, q = torch.randn(n, Hkv, D, generator=g), torch.randn(n, Hkv, D, generator=g), torch.randn(t, H, D, generator=g)
+    v[before + 5, 0, 3] = float("inf")
+    v[before + 6, 0, D - 1] = float("-inf")
+    v[before + 18, 1, 0] = float("nan")
+    v[before + t - 1, 1, 7] = float("inf")
+    k[before + 21, 1, 2] = float("nan")
+    cache.register_seq("s", 50)
+    for _ in range(-(-n // 16)):
+        cache.alloc_block("s", bm)
+    for lo, hi in ((0, before), (before, n)):
+        if hi > lo:
+            cache.write_batch(0, ["s"], [hi - lo], k[lo:hi].cuda(), v[lo:hi].cuda())
+    got = cache.attention_batch(0, ["s"], [t], q.cuda()).cpu().double()
+    for i in range(t):
+        want = _ref(q[i:i + 1], k[:before + i + 1], v[:before + i + 1], H, Hkv, "grouped", before + i)[0]
+        fin = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got[i]), fin), i
+        assert (got[i][fin] - want[fin]).abs().max() <= 1e-5, i
+        inf = torch.isinf(want)
+        assert torch.equal(got[i][inf], want[inf]), i

@@ -631,7 +631,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     // Attention of T tiles of query rows (qf) over pages [page0, page0 + np)
     // of table `trow` for kv-head kvh; tokens at positions >= row_len[t] are
     // masked for this lane's row of tile t, and V rows at or past len (the
-    // longest) are zeroed.
+    // longest) are zeroed; every row sees the tokens before `open`.
     // trow points at the table entry of page page0; blk0 holds the block ids
     // of the first kDescPages pages.
     // Leaves O^T (o), the rows' reference max (m) and sum (l, all 4 lane
@@ -641,7 +641,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     // written into the page's LDS copy once that has landed, and to the pools
     // at byte offset row_dst of the K / V pool.
     auto attend = [&]<int T>(const qfrag_t (&qf)[T][KK], const int32_t *trow, int4 blk0, int page0, int np, int len,
-                             const int (&row_len)[T], int kvh, float sl2, f32x4 (&o)[DT][T], float (&m)[T], float (&l)[T], int fuse_tib,
+                             const int (&row_len)[T], int open, int kvh, float sl2, f32x4 (&o)[DT][T], float (&m)[T], float (&l)[T], int fuse_tib,
                              u32x4 nrow, size_t row_dst) {
         const char *kbase = p.k_pool + ((size_t)kvh * PAGE);
         const char *vbase = p.v_pool + ((size_t)kvh * PAGE);
@@ -661,7 +661,8 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[dt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        auto page = [&](int pi, int s) {
+        // SOME: a row group's page with tokens that only some of its rows see
+        auto page = [&]<bool SOME>(int pi, int s) {
             wait_page(pi, np);
             if constexpr (KV == ZK_BF16) {
                 if (fuse_tib >= 0 && pi == np - 1) {  // the step's token over the page's stale row
@@ -770,6 +771,18 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
                         for (int j = 0; j < VW; ++j) w[i][j] = 0u;
             }
+            // V of a token must not reach the rows that do not see it, whose
+            // weight of 0 times an infinity would be NaN: a page with a value that
+            // is not finite takes its tokens one by one.
+            bool one_by_one = false;
+            if constexpr (SOME) {
+                uint32_t top = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < VW; ++j) top = max(top, w[i][j] & 0x7f800000u);
+                one_by_one = __builtin_amdgcn_ballot_w64(top == 0x7f800000u) != 0;
+            }
             s16x4 va[F32 ? 1 : DT];  // element i of tile dt = V[4*grp+i][DT*col+dt]
             if constexpr (!F32)
 #pragma unroll
@@ -803,6 +816,23 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) pr[i] = exp2_fast(sc[i] - m[t]);
                 l[t] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+                if constexpr (SOME) {
+                    if (one_by_one) {
+#pragma unroll 1
+                        for (int g = 0; g < 4; ++g)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const bool sees = (page0 + pi) * BS + 4 * g + i < row_len[t];
+#pragma unroll
+                                for (int dt = 0; dt < DT; ++dt) {
+                                    const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                        grp == g ? __uint_as_float(w[i][dt]) : 0.0f, pr[i], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                                    if (sees) o[dt][t] += c;
+                                }
+                            }
+                        continue;
+                    }
+                }
                 if constexpr (F32) {
                     // k-step i: V^T column token 4*grp+i (A) and its weight (B)
 #pragma unroll
@@ -835,7 +865,12 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         if constexpr (!DIRECT)
             if (np <= kStages) claim_next();
         // one page per iteration (a single loop-carried accumulator set)
-        for (int pi = 0, st = 0; pi < np; ++pi, st = (st + 1 == kStages ? 0 : st + 1)) page(pi, st);
+        // (row groups: the pages that every row sees whole first)
+        const int whole = ROWS ? min(np, max(0, open / BS - page0)) : np;
+        int pi = 0, st = 0;
+        for (; pi < whole; ++pi, st = (st + 1 == kStages ? 0 : st + 1)) page.template operator()<false>(pi, st);
+        if constexpr (ROWS)
+            for (; pi < np; ++pi, st = (st + 1 == kStages ? 0 : st + 1)) page.template operator()<true>(pi, st);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             l[t] += xor16(l[t]);
@@ -901,7 +936,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         float m[2], l[2];
         const int all[2] = {0x7fffffff, 0x7fffffff};
         attend.template operator()<2>(qf, p.bt + (size_t)n0 * p.max_blocks + page0, d1, page0, np, 0x7fffffff, all,
-                                      kvh, p.scale_log2, o, m, l, -1, no_row, 0);
+                                      0x7fffffff, kvh, p.scale_log2, o, m, l, -1, no_row, 0);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int r = 16 * t + col;
@@ -946,7 +981,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         f32x4 o[DT][1];
         const int own_len[1] = {len};
         float m[1], l[1];
-        attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, own_len, kvh, sl2,
+        attend.template operator()<1>(qf, p.bt + (size_t)n * p.max_blocks + page0, d1, page0, np, len, own_len, len, kvh, sl2,
                                       o, m, l, fuse_tib, nrow, row_dst);
         if (col < G) {
             if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
@@ -1018,7 +1053,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         }
         f32x4 o[DT][2];
         float m[2], l[2];
-        attend.template operator()<2>(qf, row, first, page0, np, len, row_len, kvh, p.scale_log2, o, m, l, -1, no_row, 0);
+        attend.template operator()<2>(qf, row, first, page0, np, len, row_len, d.w, kvh, p.scale_log2, o, m, l, -1, no_row, 0);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int r = 16 * t + col, qh = qhead_of(p, kvh, r % G, G);
