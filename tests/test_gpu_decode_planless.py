@@ -66,3 +66,37 @@ def test_f32_operands_off_their_alignment():
     for qq, kk, vv in ((off(q), to_dev(kp), to_dev(vp)), (to_dev(q), off(kp), off(vp))):
         out = ops.paged_decode(qq, kk, vv, *args)
         assert max_abs_err(to_host(out), ref) <= TOL[oracle.F32]
+
+
+@pytest.mark.parametrize("dt", [oracle.F32, oracle.BF16])
+@pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (8, 8, 128), (16, 8, 64)])
+def test_pages_of_minus_infinity(dt, H, Hkv, D):
+    """Keys whose scores are all -inf (whole pages, whole partitions, at the
+    start, inside and at the end of a partition) have weight 0; a context of
+    nothing else is NaN, as a softmax of it is; an empty one is zeros."""
+    dead = {0: [(0, 16)], 1: [(0, 2 * PART)], 2: [(PART, PART + 40)], 3: [(PART, 2 * PART), (4 * PART - 16, 4 * PART)],
+            4: [(0, 5 * PART + 3)], 5: [(0, 90)], 7: [(0, 26 * PART - 1)]}
+    lens = [40, 5 * PART + 3, 5 * PART + 3, 5 * PART + 3, 5 * PART + 3, 90, 0, 26 * PART]
+    q, kp, vp, bt, _ = decode_case(980 + H + D, H, Hkv, D, lens, dt)
+    qf = as_f32(q, dt).copy()
+    qf[:, :, 0] = np.abs(qf[:, :, 0]) + 0.5
+    q = qf if dt == oracle.F32 else oracle.bf16_bits_from_f32(qf).reshape(qf.shape)
+    for n, spans in dead.items():
+        for lo, hi in spans:
+            for t in range(lo, hi):
+                kp[bt[n, t // 16], :, t % 16, 0] = -np.inf if dt == oracle.F32 else 0xff80
+    got = _decode(q, kp, vp, bt, lens)
+    kf, vf, qf = (as_f32(x, dt).astype(np.float64) for x in (kp, vp, q))
+    for n, length in enumerate(lens):
+        alive = np.ones(length, bool)
+        for lo, hi in dead.get(n, []):
+            alive[lo:hi] = False
+        if not alive.any():
+            assert np.isnan(got[n]).all() if length else np.all(got[n] == 0)
+            continue
+        t = np.flatnonzero(alive)
+        for h in range(H):
+            k, v = (x[bt[n, t // 16], h // (H // Hkv), t % 16] for x in (kf, vf))
+            w = k @ qf[n, h] / np.sqrt(D)
+            w = np.exp(w - w.max())
+            assert max_abs_err(got[n, h], w @ v / w.sum()) <= TOL[dt], (n, h)

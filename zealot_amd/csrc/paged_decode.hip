@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -656,7 +657,9 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         };
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            m[t] = -INFINITY;
+            // planless and f32: finite, so that keys whose scores are -inf have
+            // weight 0 and not NaN wherever a partition begins
+            m[t] = DIRECT || F32 ? -FLT_MAX : -INFINITY;
             l[t] = 0.0f;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[dt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -875,6 +878,12 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         for (int t = 0; t < T; ++t) {
             l[t] += xor16(l[t]);
             l[t] += xor32(l[t]);
+            if constexpr (DIRECT || F32) {
+                if (l[t] == 0.0f) {  // no weights: no keys, or scores of -inf only (NaN if nothing else comes)
+                    m[t] = -INFINITY;
+                    if (np > 0) l[t] = NAN;
+                }
+            }
         }
     };
 
@@ -985,7 +994,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                                       o, m, l, fuse_tib, nrow, row_dst);
         if (col < G) {
             if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
-                const float inv = l[0] > 0.0f ? vscale / l[0] : 0.0f;
+                const float inv = l[0] == 0.0f ? 0.0f : vscale / l[0];
                 const size_t ob = (qr * H + qh) * D;
                 if (p.q_f32) {
                     f32x4 o2[DT][2];
@@ -1063,7 +1072,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 store_partial(((size_t)(g * NT + r / G) * H + qh) * p.max_parts + part, o, t, 1.0f, m[t], l[t]);
                 continue;
             }
-            const float inv = l[t] > 0.0f ? 1.0f / l[t] : 0.0f;
+            const float inv = l[t] == 0.0f ? 0.0f : 1.0f / l[t];
             const size_t ob = ((size_t)(d.y + r / G) * H + qh) * D;
             if (p.q_f32) {
                 store_row_f32((float *)p.out + ob, o, t, inv);
@@ -1344,6 +1353,18 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kernel(Params p) {
         if (lane + 64 * c < D) store_out(p, (qrow(p, n) * p.num_heads + h) * D + lane + 64 * c, acc[c] * inv);
 }
 
+// A partition's sum of weights without its mark.  One without weights (m =
+// -inf) counts nothing: its l may be NaN.
+__device__ __forceinline__ float sum_of(float2 ml) { return ml.x == -INFINITY ? 0.0f : fabsf(ml.y); }
+
+// 1 / L where no partition has weight: 0 (no keys), or NaN where one had keys
+// with scores of -inf only (its l is NaN, and counts here alone).
+__device__ __forceinline__ float without_weights(const Params &p, size_t base, int nparts) {
+    float sum = 0.0f;
+    for (int i = 0; i < nparts; ++i) sum += fabsf(p.ml[base + i].y);
+    return sum;
+}
+
 // The same merge for D = 4 * LP (D in {64, 128, 256}): LP lanes hold a
 // partition's partial output as one float4 each, so one load instruction
 // covers 64 / LP partitions and all of a sequence's partitions are in flight
@@ -1378,13 +1399,13 @@ __global__ void __launch_bounds__(kWave) decode_reduce_vec_kernel(Params p) {
     for (int i = lane + kWave; i < nparts; i += kWave) M = fmaxf(M, p.ml[base + i].x);
     for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
     auto weight = [&](float2 v) { return v.x == -INFINITY ? 0.0f : exp2f(v.x - M); };
-    float L = ml0.y * weight(ml0);
+    float L = sum_of(ml0) * weight(ml0);
     for (int i = lane + kWave; i < nparts; i += kWave) {
         const float2 v = p.ml[base + i];
-        L += v.y * weight(v);
+        L += sum_of(v) * weight(v);
     }
     for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < nparts; c0 += kWave) {  // weights of partitions c0 .. c0 + 63 in lanes
         const float w = weight(c0 == 0 ? ml0 : (c0 + lane < nparts ? p.ml[base + c0 + lane] : none));
@@ -1478,7 +1499,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     for (int i = 0; i < C; ++i)
         if (i < nparts) {
             const float w = weight(ml[i]);
-            L += ml[i].y * w;
+            L += sum_of(ml[i]) * w;
 #pragma unroll
             for (int k = 0; k < F4; ++k)
 #pragma unroll
@@ -1487,7 +1508,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     for (int i = C; i < nparts; ++i) {
         const float2 v = p.ml[base + i];
         const float w = weight(v);
-        L += (MARKS ? fabsf(v.y) : v.y) * w;
+        L += sum_of(v) * w;
 #pragma unroll
         for (int k = 0; k < F4; ++k) {
             const f32x4 y = *reinterpret_cast<const f32x4 *>(p.po + (base + i) * D + d0 + 4 * k);
@@ -1495,7 +1516,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
             for (int c = 0; c < 4; ++c) acc[k][c] = fmaf(w, y[c], acc[k][c]);
         }
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
     const size_t ob = (qrow(p, n) * p.num_heads + qh) * D + d0;
     if (p.q_f32) {
 #pragma unroll
@@ -1547,7 +1568,7 @@ __global__ void __launch_bounds__(256) decode_reduce_many_kernel(Params p) {
     float L = 0.0f;
     for (int i = lane; i < nparts; i += kWave) {
         const float2 v = p.ml[base + i];
-        L += fabsf(v.y) * weight(v.x);
+        L += sum_of(v) * weight(v.x);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
@@ -1572,7 +1593,7 @@ __global__ void __launch_bounds__(256) decode_reduce_many_kernel(Params p) {
     acc = part_sum[t];
 #pragma unroll
     for (int q = 1; q < PG; ++q) acc += part_sum[q * LP + t];
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
     const size_t ob = (qrow(p, n) * p.num_heads + h) * D + d0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) store_out(p, ob + c, acc[c] * inv);
