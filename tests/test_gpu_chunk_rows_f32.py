@@ -125,3 +125,47 @@ def test_rows_do_not_see_later_tokens_infinities(H, Hkv, D, before, t):
         assert (got[i][fin] - want[fin]).abs().max() <= 1e-5, i
         inf = torch.isinf(want)
         assert torch.equal(got[i][inf], want[inf]), i
+
+
+def test_more_rows_than_one_grid_holds():
+    """66000 rows of one chunk in several partitions: more than the 65535 that
+    a launch of the merge takes; rows from all over the chunk against float64."""
+    from zealot_amd import BlockManager, KVCache
+    H, D, t = 1, 64, 66000
+    pages = -(-t // 16)
+    bm = BlockManager(pages, 16)
+    cache = KVCache(pages, 16, 1, H, D, dtype=torch.float32, max_seqs=1, max_blocks_per_seq=pages)
+    cache.register_seq("s", pages)
+    for _ in range(pages):
+        cache.alloc_block("s", bm)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    k, v, q = (torch.randn((t, H, D), generator=g, device="cuda") for _ in range(3))
+    cache.write_batch(0, ["s"], [t], k, v)
+    got = cache.attention_batch(0, ["s"], [t], q)
+    for i in (0, 31, 32, 16383, 16384, 40000, 65503, 65504, 65534, 65535, 65536, t - 1):
+        w = torch.softmax(k[:i + 1, 0].double() @ q[i, 0].double() / math.sqrt(D), 0)
+        assert (got[i, 0].double() - w @ v[:i + 1, 0].double()).abs().max() <= 1e-5, i
+
+
+def test_rows_of_one_partition_take_no_partials():
+    """8192 rows whose contexts are one partition each: no space for partials
+    (a slot a row and head would be 140 MB)."""
+    from zealot_amd import BlockManager, KVCache
+    H, Hkv, D, t = 32, 8, 128, 8192
+    bm = BlockManager(t // 16, 16)
+    cache = KVCache(t // 16, 16, 1, Hkv, D, dtype=torch.float32, max_seqs=1, max_blocks_per_seq=t // 16)
+    cache.register_seq("s", t // 16)
+    for _ in range(t // 16):
+        cache.alloc_block("s", bm)
+    kv = torch.randn((t, Hkv, D), device="cuda")
+    q = torch.randn((t, H, D), device="cuda")
+    out = torch.empty_like(q)
+    cache.write_batch(0, ["s"], [t], kv, kv)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    cache.attention_batch(0, ["s"], [t], q, out=out)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 32 << 20
+    for i in (0, 4095, t - 1):
+        w = torch.softmax(kv[:i + 1, 0].double() @ q[i, 0].double() / math.sqrt(D), 0)
+        assert (out[i, 0].double() - w @ kv[:i + 1, 0].double()).abs().max() <= 1e-5, i

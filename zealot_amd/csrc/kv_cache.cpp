@@ -1383,9 +1383,9 @@ int chunk_rows_f32(zk_kv_cache *c, size_t layer, const std::vector<const SeqStat
             *g++ = make_int4((int)i, (int)(off[i] + t), std::min(nt, len[i] - t), start + t + 1);
     }
     if (int rc = put(c, c->d_pre, host.data(), host.size(), "KVCache chunk rows")) return rc;
-    // groups of one launch: its grid's limit
-    for (size_t g0 = 0; g0 < groups; g0 += 65535) {
-        const int gn = (int)std::min<size_t>(65535, groups - g0);
+    const size_t most = (size_t)zk::paged_rows_max_groups(num_heads, (int)c->num_kv_heads);
+    for (size_t g0 = 0; g0 < groups; g0 += most) {
+        const int gn = (int)std::min(most, groups - g0);
         const size_t ws = zk::paged_rows_workspace(gn, num_heads, (int)c->num_kv_heads, (int)c->head_dim, (int)stride);
         if (int rc = c->d_pws.ensure(ws, "KVCache chunk rows workspace")) return rc;
         char *d = (char *)c->d_pre.dev.p;

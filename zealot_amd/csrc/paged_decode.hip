@@ -2093,8 +2093,12 @@ void launch_rows(const Params &p, int groups, hipStream_t s, int G) {
 }  // namespace
 
 size_t zk::paged_rows_workspace(int groups, int num_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq) {
+    if (rows_parts(groups, num_kv_heads, max_blocks_per_seq) == 1) return 256;  // every row is written by its own item
     return rows_layout(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq).total;
 }
+
+// The attention's grid holds a group and the merge's a row per z / y: 65535 at most.
+int zk::paged_rows_max_groups(int num_heads, int num_kv_heads) { return 65535 / (32 * num_kv_heads / num_heads); }
 
 int zk::paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, void *out,
                    const int32_t *block_tables, const int4 *row_groups, int groups, int num_heads, int num_kv_heads,
@@ -2107,7 +2111,9 @@ int zk::paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const vo
     if (!q || !k_pool || !v_pool || !out || !block_tables || !row_groups || !workspace)
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged rows: NULL pointer");
     const WsLayout w = rows_layout(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq);
-    if (groups > 65535 || workspace_bytes < w.total || ((uintptr_t)workspace & 255u))
+    if (groups > paged_rows_max_groups(num_heads, num_kv_heads) ||
+        workspace_bytes < paged_rows_workspace(groups, num_heads, num_kv_heads, head_dim, max_blocks_per_seq) ||
+        ((uintptr_t)workspace & 255u))
         return set_error(ZK_ERR_INVALID_ARGUMENT, "Internal error: paged rows: too many groups or workspace too small");
     const int G = num_heads / num_kv_heads;
     Params p{};

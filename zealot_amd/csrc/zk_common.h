@@ -126,6 +126,7 @@ int paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const void
 // row, tokens (at most 32 / G), context of its first token}; token i attends its
 // first w + i tokens.  Tables must be valid up to every length.
 bool paged_rows_supported(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
+int paged_rows_max_groups(int num_heads, int num_kv_heads);  // of one call
 size_t paged_rows_workspace(int groups, int num_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq);
 int paged_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, void *out,
                const int32_t *block_tables, const int4 *row_groups, int groups, int num_heads, int num_kv_heads,
