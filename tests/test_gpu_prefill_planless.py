@@ -50,3 +50,24 @@ def test_planned_launch_with_cuts():
     chunks = [int(x) for x in rng.integers(30, 90, 60)]
     starts = [int(x) for x in rng.integers(0, 100, 60)]
     _check(32, 32, 64, starts, chunks, cuts={3: 0, 10: 1, 33: 2})
+
+
+@pytest.mark.parametrize("start,chunk,best", [(0, 40, 11), (1500, 33, 3), (1500, 33, 1100), (1500, 33, 1510), (2000, 33, None)])
+def test_scores_far_below_zero(start, chunk, best):
+    """Scores of some -1e31 (powers of two, so that scaling them is exact) have the
+    weights their differences give, with one split and with several: key `best`
+    alone, or all the same."""
+    H, Hkv, D = 8, 2, 128
+    q, kp, vp, _, bt, cu, _, _ = _case(340, H, Hkv, D, [start], [chunk], "bf16")
+    bits = oracle.bf16_bits_from_f32
+    q[:, :, 0] = bits(np.full((1,), 2.0**40, np.float32))[0]
+    kp[:, :, :, 0] = bits(np.full((1,), -2.0**67, np.float32))[0]
+    if best is not None:
+        kp[bt[0, best // 16], :, best % 16, 0] = bits(np.full((1,), -2.0**66, np.float32))[0]
+    out = as_f32(_run(q, kp, vp, bt, cu, [start], True, "grouped", None, None), oracle.BF16)
+    t = np.arange(start + chunk)
+    v = as_f32(vp, oracle.BF16)[bt[0, t // 16], :, t % 16]  # [tokens, Hkv, D]
+    for i in range(chunk):
+        seen = start + i + 1
+        want = v[best] if best is not None and best < seen else v[:seen].mean(0, dtype=np.float64)
+        assert max_abs_err(out[i].reshape(Hkv, H // Hkv, D), want[:, None]) <= 2e-2, i

@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <climits>
 #include <cmath>
 #include <cstdint>
@@ -68,7 +69,7 @@ constexpr int kXcds = 8;                         // XCDs of an MI355X
 constexpr int kXcdBins = kMaxBins / kXcds;       // longest-first bins per XCD queue
 constexpr int kQueueStride = 32;                 // ints between XCD queue heads (128 B)
 constexpr float kRescaleSlack = 8.0f;  // lazy-rescale slack, log2 units
-constexpr float kNoKeyMax = -1e30f;    // reference max of a row that has seen no key yet
+constexpr float kNoKeyMax = -FLT_MAX;  // reference max of a row that has seen no key yet: below every score
 constexpr int kMaxSplits = 16;         // key splits of a planless item
 
 struct PParams {
@@ -667,7 +668,8 @@ prefill_mfma_kernel(PParams p) {
                 m[t] = fmaxf(cm, xor32(cm));
                 // a later split's first keys may all lie past a row's limit:
                 // a finite reference keeps its weights 0 and not NaN
-                if constexpr (DIRECT) m[t] = fmaxf(m[t], kNoKeyMax);
+                if constexpr (DIRECT)
+                    if (p0 > 0) m[t] = fmaxf(m[t], kNoKeyMax);
             }
         }
         // Iteration j: the weights of pair j (P) go through PV while pair
