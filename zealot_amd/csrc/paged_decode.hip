@@ -1668,10 +1668,18 @@ void launch_mfma_k(const Params &p, hipStream_t s) {
             const dim3 grid(p.num_kv_heads, p.num_sg * p.shared_parts + p.num_seqs * own);
             decode_mfma_kernel<KV, D, G, true, false, true><<<grid, kWave, 0, s>>>(p);
         }
-    } else if (p.num_waves > 0)
+    } else if (p.num_waves > 0) {
         decode_mfma_kernel<KV, D, G, false><<<p.num_waves, kWave, 0, s>>>(p);
-    else
-        decode_mfma_kernel<KV, D, G, true><<<dim3(p.num_kv_heads, p.max_parts, p.num_seqs), kWave, 0, s>>>(p);
+    } else {
+        // Not a multiple of four partitions a sequence: a table wider than the
+        // contexts leaves a sequence's later workgroups without work, and at a
+        // stride of 20, say, those with work go to 8 of an XCD's 32 CUs (40 x
+        // 100..1000 tokens, tables of 1024 pages: 50 us, 33.6 with 21; 128 x
+        // 200..2000 in their own tables 121 and 109; two partitions as three, six
+        // as seven, and f32's one wave a SIMD, lose as often as they win).
+        const int parts = p.max_parts + (KV != ZK_F32 && p.max_parts % 4 == 0);
+        decode_mfma_kernel<KV, D, G, true><<<dim3(p.num_kv_heads, parts, p.num_seqs), kWave, 0, s>>>(p);
+    }
 }
 
 template <int KV, int D>
