@@ -148,8 +148,10 @@ struct Params {
 // Tokens of a row group: its tile of 32 rows holds the G heads of each.
 __device__ __forceinline__ int group_tokens(const Params &p) { return 32 * p.num_kv_heads / p.num_heads; }
 
+// PLANLESS launches alone have groups.
+template <bool PLANLESS = false>
 __device__ __forceinline__ size_t qrow(const Params &p, int n) {
-    if (p.groups) return (size_t)p.groups[n / group_tokens(p)].y + n % group_tokens(p);
+    if (PLANLESS && p.groups) return (size_t)p.groups[n / group_tokens(p)].y + n % group_tokens(p);
     return p.q_rows ? (size_t)p.q_rows[n] : (size_t)n;
 }
 
@@ -243,6 +245,12 @@ __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_ex
 __device__ __forceinline__ uint32_t bf16x2_rne(float lo, float hi) {
     typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2_t));
+}
+
+// scale / l for a row of maximum m: 0 where it saw no keys (m = -inf), NaN where
+// all their scores were -inf (l = 0 at the lowest finite m).
+__device__ __forceinline__ float inverse_sum(float l, float m, float scale = 1.0f) {
+    return l > 0.0f ? scale / l : m == -INFINITY ? 0.0f : NAN;
 }
 
 // Lazy-rescale slack of the shared-prefix softmax, in log2 units.
@@ -442,6 +450,9 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
     constexpr int BS = 16;
     constexpr int BIDS = DIRECT && !ROWS ? kDirectPages : kMaxItemPages;
     constexpr bool F32 = KV == ZK_F32;
+    // The maximum starts finite, so that keys whose scores are -inf have weight
+    // 0 and not NaN wherever a partition begins (fp8 keys are finite).
+    constexpr bool LOWEST = DIRECT || KV != ZK_FP8_E4M3;
     constexpr int ELT = F32 ? 4 : KV == ZK_BF16 ? 2 : 1;
     constexpr int DG = D / 4;            // head dims per lane group in QK
     constexpr int KK = F32 ? D / 16 : DG / 8;  // 16-byte Q chunks per lane (bf16: MFMA k-steps)
@@ -657,9 +668,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         };
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            // planless and f32: finite, so that keys whose scores are -inf have
-            // weight 0 and not NaN wherever a partition begins
-            m[t] = DIRECT || F32 ? -FLT_MAX : -INFINITY;
+            m[t] = LOWEST ? -FLT_MAX : -INFINITY;
             l[t] = 0.0f;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[dt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -878,12 +887,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
         for (int t = 0; t < T; ++t) {
             l[t] += xor16(l[t]);
             l[t] += xor32(l[t]);
-            if constexpr (DIRECT || F32) {
-                if (l[t] == 0.0f) {  // no weights: no keys, or scores of -inf only (NaN if nothing else comes)
-                    m[t] = -INFINITY;
-                    if (np > 0) l[t] = NAN;
-                }
-            }
+            if (LOWEST && np == 0) m[t] = -INFINITY;
         }
     };
 
@@ -994,7 +998,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                                       o, m, l, fuse_tib, nrow, row_dst);
         if (col < G) {
             if (ns == 0 && nparts <= 1) {  // the whole context: write the output row
-                const float inv = l[0] == 0.0f ? 0.0f : vscale / l[0];
+                const float inv = inverse_sum(l[0], m[0], vscale);
                 const size_t ob = (qr * H + qh) * D;
                 if (p.q_f32) {
                     f32x4 o2[DT][2];
@@ -1072,7 +1076,7 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 store_partial(((size_t)(g * NT + r / G) * H + qh) * p.max_parts + part, o, t, 1.0f, m[t], l[t]);
                 continue;
             }
-            const float inv = l[t] == 0.0f ? 0.0f : 1.0f / l[t];
+            const float inv = inverse_sum(l[t], m[t]);
             const size_t ob = ((size_t)(d.y + r / G) * H + qh) * D;
             if (p.q_f32) {
                 store_row_f32((float *)p.out + ob, o, t, inv);
@@ -1353,18 +1357,6 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kernel(Params p) {
         if (lane + 64 * c < D) store_out(p, (qrow(p, n) * p.num_heads + h) * D + lane + 64 * c, acc[c] * inv);
 }
 
-// A partition's sum of weights without its mark.  One without weights (m =
-// -inf) counts nothing: its l may be NaN.
-__device__ __forceinline__ float sum_of(float2 ml) { return ml.x == -INFINITY ? 0.0f : fabsf(ml.y); }
-
-// 1 / L where no partition has weight: 0 (no keys), or NaN where one had keys
-// with scores of -inf only (its l is NaN, and counts here alone).
-__device__ __forceinline__ float without_weights(const Params &p, size_t base, int nparts) {
-    float sum = 0.0f;
-    for (int i = 0; i < nparts; ++i) sum += fabsf(p.ml[base + i].y);
-    return sum;
-}
-
 // The same merge for D = 4 * LP (D in {64, 128, 256}): LP lanes hold a
 // partition's partial output as one float4 each, so one load instruction
 // covers 64 / LP partitions and all of a sequence's partitions are in flight
@@ -1399,13 +1391,13 @@ __global__ void __launch_bounds__(kWave) decode_reduce_vec_kernel(Params p) {
     for (int i = lane + kWave; i < nparts; i += kWave) M = fmaxf(M, p.ml[base + i].x);
     for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
     auto weight = [&](float2 v) { return v.x == -INFINITY ? 0.0f : exp2f(v.x - M); };
-    float L = sum_of(ml0) * weight(ml0);
+    float L = ml0.y * weight(ml0);
     for (int i = lane + kWave; i < nparts; i += kWave) {
         const float2 v = p.ml[base + i];
-        L += sum_of(v) * weight(v);
+        L += v.y * weight(v);
     }
     for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
-    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
+    const float inv = inverse_sum(L, M);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < nparts; c0 += kWave) {  // weights of partitions c0 .. c0 + 63 in lanes
         const float w = weight(c0 == 0 ? ml0 : (c0 + lane < nparts ? p.ml[base + c0 + lane] : none));
@@ -1499,7 +1491,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     for (int i = 0; i < C; ++i)
         if (i < nparts) {
             const float w = weight(ml[i]);
-            L += sum_of(ml[i]) * w;
+            L += ml[i].y * w;
 #pragma unroll
             for (int k = 0; k < F4; ++k)
 #pragma unroll
@@ -1508,7 +1500,7 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
     for (int i = C; i < nparts; ++i) {
         const float2 v = p.ml[base + i];
         const float w = weight(v);
-        L += sum_of(v) * w;
+        L += (MARKS ? fabsf(v.y) : v.y) * w;
 #pragma unroll
         for (int k = 0; k < F4; ++k) {
             const f32x4 y = *reinterpret_cast<const f32x4 *>(p.po + (base + i) * D + d0 + 4 * k);
@@ -1516,8 +1508,8 @@ __global__ void __launch_bounds__(kWave) decode_reduce_kv_kernel(Params p) {
             for (int c = 0; c < 4; ++c) acc[k][c] = fmaf(w, y[c], acc[k][c]);
         }
     }
-    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
-    const size_t ob = (qrow(p, n) * p.num_heads + qh) * D + d0;
+    const float inv = inverse_sum(L, M);
+    const size_t ob = (qrow<MARKS>(p, n) * p.num_heads + qh) * D + d0;
     if (p.q_f32) {
 #pragma unroll
         for (int k = 0; k < F4; ++k) {
@@ -1568,7 +1560,7 @@ __global__ void __launch_bounds__(256) decode_reduce_many_kernel(Params p) {
     float L = 0.0f;
     for (int i = lane; i < nparts; i += kWave) {
         const float2 v = p.ml[base + i];
-        L += sum_of(v) * weight(v.x);
+        L += fabsf(v.y) * weight(v.x);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
@@ -1593,8 +1585,8 @@ __global__ void __launch_bounds__(256) decode_reduce_many_kernel(Params p) {
     acc = part_sum[t];
 #pragma unroll
     for (int q = 1; q < PG; ++q) acc += part_sum[q * LP + t];
-    const float inv = L != 0.0f ? 1.0f / L : without_weights(p, base, nparts);
-    const size_t ob = (qrow(p, n) * p.num_heads + h) * D + d0;
+    const float inv = inverse_sum(L, M);
+    const size_t ob = (qrow<true>(p, n) * p.num_heads + h) * D + d0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) store_out(p, ob + c, acc[c] * inv);
 }
