@@ -1281,7 +1281,7 @@ int decode_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState 
                               (int)c->head_dim, (int)c->block_size, (int)stride, (int64_t)c->num_blocks, scale,
                               mapping, dks, dvs, c->d_ws.p, c->d_ws.cap, c->stream, nsg ? &pg : nullptr, drows,
                               q_stride, /*trusted_tables=*/true,  // built from the sequences' handles
-                              reuse, append, &c->dec_head_set, max_waves);
+                              reuse, append, &c->dec_head_set, max_waves, (int)std::min<size_t>(c->num_layers, 1024));
     if (rc == ZK_OK) c->plan_sig = std::move(sig);
     return rc;
 }

@@ -1761,6 +1761,13 @@ int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves)
 // 22 / 15, 64 x 512..8192 bf16 177 / 165, fp8 116 / 89, f32 324 / 313; 40 x
 // 1024..16384 206 / 193; then 192 x 300..4000 bf16 264 / 278 and 256 x 512..8192
 // 643 / 708: the line lies at 3 GB of capacity.
+// Where one plan serves the layers of a step (plan_launches) and the tables need
+// no walk, nothing of that is saved, and the line lies where the kernels' own
+// times cross (planned / planless, us a layer with the merge; 8 layers): bf16 96 x
+// 200..2000 (0.8 GB) 94 / 83, 48 x 512..8192 (1.6) 135 / 127, 256 x 100..1000 (1.1)
+// 117 / 119, 64 x 512..8192 (2.1) 176.4 / 178.9, 88 x (3.0) 237 / 246; fp8 48 x
+// 4000..16000 (1.6) 188 / 176, 110 x 512..8192 (1.8) 171 / 170; f32 24 x 512..4096
+// (0.8) 88 / 75, 64 x 100..2000 (1.0) 101 / 113, 8 x 4000..16000 (1.0) 122 / 133.
 //
 // The partition length P balances the items' fixed cost, (units / P) a / waves,
 // against the tail of one item, P b: P ~ sqrt(units), with page_bytes for the
@@ -1769,17 +1776,25 @@ int shared_part_pages_for(long total_shared_pages, int num_kv_heads, long waves)
 // than 8 pages do not pay for the reduce; the count is rounded to the nearest
 // so that a table a little over P stays one partition (no reduce at all).
 constexpr double kDirectBytes = 3e9;
+constexpr int kPlanLaunches = 4;  // a plan over fewer launches still costs each 5 us and more
+double direct_limit(int kv_dtype, int plan_launches) {
+    if (plan_launches < kPlanLaunches) return kDirectBytes;
+    return kv_dtype == ZK_F32 ? 0.9e9 : kv_dtype == ZK_BF16 ? 1.6e9 : 2.0e9;
+}
 // Shared prefixes without a plan: about this many shared items over all
 // kv-heads (each streams its pages for up to 32 rows, beside the sequences' own
 // one- and two-page items, all resident at once), of at least 10 pages.  Against
 // the planned launch (eight queues, 32-page items), four layers of a step, us: 16
 // x 8 forks of 2050 tokens 152 / 139, 12 x 8 of 3900 187 / 172, 5 x 11 of 2420 117 /
 // 107, 8 x 2 of 700 76 / 62, 1 x 2 of 400 70 / 45; 256, 512, 640 and 1024 items 171,
-// 146, 147 and 161 on the first.
+// 146, 147 and 161 on the first.  Over 8 layers with one plan, us a layer: 8 x 8 of
+// 4000 (131 MB of shared pages) 40.5 / 36, 24 x 8 of 4000 (393) 97 / 97, 16 x 8 of
+// 8000 (525) 125 / 132, 8 x 8 of 16000 (523) 121 / 130, 200 x 4 of 1000 (817) 196 / 211.
 constexpr long kSharedItems = 384, kSharedMinPages = 10;
-int direct_parts(double units, double page_bytes, int max_blocks) {
+constexpr double kDirectSharedBytes = 0.45e9;
+int direct_parts(double units, double page_bytes, int max_blocks, double limit = kDirectBytes) {
     const double bytes = units * page_bytes;
-    if (bytes > kDirectBytes) return 0;
+    if (bytes > limit) return 0;
     const double pp = std::min((double)kDirectPages, std::max(8.0, std::sqrt(bytes) * 1e-3));
     return std::max((max_blocks + kDirectPages - 1) / kDirectPages, std::max(1, (int)(max_blocks / pp + 0.5)));
 }
@@ -1843,10 +1858,10 @@ struct DecodeShape {
     WsLayout w;
 };
 // max_waves > 0 caps the MFMA path's persistent grid (partitions are sized
-// for the waves that run them).
+// for the waves that run them); plan_launches: see direct_limit.
 DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num_kv_heads, int head_dim,
                          int block_size, int max_blocks_per_seq, const PrefixGroups *pg, bool aligned,
-                         size_t workspace_bytes, int max_waves = 0) {
+                         size_t workspace_bytes, int max_waves = 0, int plan_launches = 1) {
     DecodeShape d;
     const int G = num_heads / num_kv_heads;
     // f32 pools: any alignment was and is accepted, the 16-byte accesses of
@@ -1873,15 +1888,18 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
     d.direct = false;
     d.shared_parts = 0;
     if (workspace_bytes < d.need) return d;  // refused
+    const double limit = direct_limit(kv_dtype, plan_launches);
     if (d.use_mfma && d.shared && max_waves == 0 && !part_pages_env() && pg->max_pages > 0) {
         // shared prefixes without a plan: see kSharedItems
         const double page_bytes = 2.0 * block_size * head_dim * elt_size(kv_dtype);
         const double own_units = (double)num_seqs * std::max(1, pg->max_rest) * num_kv_heads;
-        const int own = direct_parts(own_units, page_bytes, std::max(1, pg->max_rest));
+        const int own = direct_parts(own_units, page_bytes, std::max(1, pg->max_rest), limit);
+        const double shared_bytes = (double)pg->total_shared_pages * num_kv_heads * page_bytes;
         const int sp = (int)std::min<long>(kDirectPages, std::max<long>(kSharedMinPages, (pg->total_shared_pages * num_kv_heads + kSharedItems - 1) / kSharedItems));
         const int parts = (pg->max_pages + sp - 1) / sp;
         const WsLayout w = ws_layout(num_seqs, num_heads, head_dim, parts + own);
-        if (own > 0 && (own_units + (double)pg->total_shared_pages * num_kv_heads) * page_bytes <= kDirectBytes &&
+        if (own > 0 && own_units * page_bytes + shared_bytes <= limit &&
+            (plan_launches < kPlanLaunches || shared_bytes <= kDirectSharedBytes) &&
             (long)pg->num_sg * parts + (long)num_seqs * own <= 65535 && w.total <= workspace_bytes) {
             d.direct = true;
             d.waves = 0;
@@ -1894,7 +1912,7 @@ DecodeShape decode_shape(zk_dtype kv_dtype, int num_seqs, int num_heads, int num
     }
     if (d.use_mfma && !d.shared && max_waves == 0 && !part_pages_env()) {
         const int parts = direct_parts((double)num_seqs * max_blocks_per_seq * num_kv_heads,
-                                       2.0 * block_size * head_dim * elt_size(kv_dtype), max_blocks_per_seq);
+                                       2.0 * block_size * head_dim * elt_size(kv_dtype), max_blocks_per_seq, limit);
         const WsLayout w = ws_layout(num_seqs, num_heads, head_dim, parts);
         if (parts > 0 && num_seqs <= 65535 && w.total <= workspace_bytes) {
             d.direct = true;
@@ -1916,7 +1934,7 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
                      float scale, zk_gqa_mapping mapping, const float *k_scales, const float *v_scales,
                      void *workspace, size_t workspace_bytes, void *stream, const PrefixGroups *pg,
                      const int32_t *q_rows, int64_t q_stride, bool trusted_tables, bool reuse_plan,
-                     const AppendRows *append, int *head_set, int max_waves) {
+                     const AppendRows *append, int *head_set, int max_waves, int plan_launches) {
     if (int rc = check_decode_args(q_dtype, kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size,
                                    max_blocks_per_seq, num_blocks, mapping))
         return rc;
@@ -1934,7 +1952,7 @@ int zk::paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const 
     const bool aligned = (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool | (uintptr_t)out) & 15u) == 0 &&
                          q_stride % 4 == 0;
     const DecodeShape ds = decode_shape(kv_dtype, num_seqs, num_heads, num_kv_heads, head_dim, block_size,
-                                        max_blocks_per_seq, pg, aligned, workspace_bytes, max_waves);
+                                        max_blocks_per_seq, pg, aligned, workspace_bytes, max_waves, plan_launches);
     const bool use_mfma = ds.use_mfma, shared = ds.shared;
     if (append && (!use_mfma || kv_dtype != ZK_BF16 || !trusted_tables || !append->k || !append->v ||
                    append->row_bytes < (int64_t)num_kv_heads * head_dim * 2 || (append->row_bytes & 15) ||

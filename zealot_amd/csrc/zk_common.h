@@ -109,7 +109,8 @@ struct PrefixGroups {
 // uses when it reuses the plan (0 after a planning launch's successor
 // flips it); null: every launch plans.  max_waves > 0 caps the persistent
 // grid of the MFMA path (0: one wave per SIMD); a plan is reused only by
-// launches with the same cap.
+// launches with the same cap.  plan_launches: how many launches a plan will
+// serve (the layers of a step), which decides from what size on one pays.
 struct AppendRows {
     const void *k, *v;
     int64_t row_bytes;
@@ -120,7 +121,8 @@ int paged_decode(const void *q, zk_dtype q_dtype, const void *k_pool, const void
                  float scale, zk_gqa_mapping mapping, const float *k_scales, const float *v_scales,
                  void *workspace, size_t workspace_bytes, void *stream, const PrefixGroups *pg,
                  const int32_t *q_rows, int64_t q_stride = 0, bool trusted_tables = false, bool reuse_plan = false,
-                 const AppendRows *append = nullptr, int *head_set = nullptr, int max_waves = 0);
+                 const AppendRows *append = nullptr, int *head_set = nullptr, int max_waves = 0,
+                 int plan_launches = 1);
 // Attention of prompt-chunk rows on f32 pools (the shapes paged_rows_supported
 // names; 16-byte aligned operands): row group g = {row of block_tables, first q
 // row, tokens (at most 32 / G), context of its first token}; token i attends its
