@@ -359,8 +359,10 @@ int zk_cache_decode_append(zk_kv_cache *c, size_t layer, const char *const *ids,
  * num_tokens[i] tokens at this layer, attended causally over its pages (row t
  * sees positions [0, layer_len - num_tokens[i] + t], attention.cu:117-121).
  * One-row entries run as one paged decode (with prefix sharing), longer ones
- * as one chunked-prefill launch (zk_paged_prefill); shapes outside the
- * prefill kernel's run every chunk row as a decode.  Replaces the runner's
+ * as one chunked-prefill launch (zk_paged_prefill); f32 pools of the prefill
+ * kernel's shapes with 16-byte aligned q and out run 32 / (H/Hkv) consecutive
+ * rows of a chunk at a time on the decode kernel, other shapes every chunk row
+ * as a decode.  Replaces the runner's
  * per-sequence paged_forward (cuda_runner.rs:438-461).  q rows are
  * q_token_stride elements apart (0 = H * D; a fused QKV output's row length
  * reads q in place); out rows are packed [rows, H, D]. */
@@ -385,8 +387,14 @@ int zk_cache_decode_sharing(zk_kv_cache *c, int *subgroups, int64_t *shared_page
  * f32 or bf16 (out has q's dtype).  The page walk stops at the first table
  * entry < 0 or >= num_blocks, as in zk_paged_decode.  Shapes: bf16 or fp8
  * pools, block_size 16, head_dim 64 or 128, H/Hkv in {1, 2, 4, 8},
- * max_blocks_per_seq <= 2048.  workspace: caller-owned, 256-B aligned, at
- * least zk_paged_prefill_workspace_size bytes.  Asynchronous on `stream`. */
+ * max_blocks_per_seq <= 2048.  workspace: caller-owned, 256-B aligned,
+ * zk_paged_prefill_workspace_size bytes.  That holds the partial rows of small
+ * batches, whose items are split over their keys: up to 68157440 bytes, and less
+ * for a large batch than for a small one (32 / 8 heads: 30 chunks of a token 66
+ * MB, 64 of 512 tokens 0.14 MB), so a caller that reuses one workspace takes the
+ * largest of its batches' or that bound.  A workspace that holds the launch's work list but
+ * not the partials is accepted, and the batch runs unsplit.  Asynchronous on
+ * `stream`. */
 size_t zk_paged_prefill_workspace_size(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads);
 int zk_paged_prefill(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool,
                      zk_dtype kv_dtype, void *out, const int32_t *block_tables,

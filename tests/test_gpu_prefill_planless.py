@@ -7,6 +7,7 @@ import math
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from tests.gpu_util import as_f32, max_abs_err
@@ -71,3 +72,28 @@ def test_scores_far_below_zero(start, chunk, best):
         seen = start + i + 1
         want = v[best] if best is not None and best < seen else v[:seen].mean(0, dtype=np.float64)
         assert max_abs_err(out[i].reshape(Hkv, H // Hkv, D), want[:, None]) <= 2e-2, i
+
+
+def test_cache_keeps_its_prefill_workspace():
+    """Steps of any chunks run in the workspace of the cache's first one: a
+    small batch may need more space than a large one."""
+    from zealot_amd import BlockManager, KVCache
+    H, Hkv, D = 32, 8, 128
+    bm = BlockManager(1200, 16)
+    cache = KVCache(1200, 16, 1, Hkv, D, dtype=torch.bfloat16, max_seqs=60, max_blocks_per_seq=20)
+    ids = [f"s{i}" for i in range(60)]
+    for sid in ids:
+        cache.register_seq(sid, 20)
+        for _ in range(20):
+            cache.alloc_block(sid, bm)
+    x = torch.randn((60 * 100, Hkv, D), device="cuda").bfloat16()
+    q = torch.randn((60 * 100, H, D), device="cuda").bfloat16()
+    out = torch.empty_like(q)
+    free = []
+    for n, chunk in ((1, 20), (30, 2), (60, 100), (3, 40), (12, 9), (60, 2)):
+        rows = n * chunk
+        cache.write_batch(0, ids[:n], [chunk] * n, x[:rows], x[:rows])
+        cache.attention_batch(0, ids[:n], [chunk] * n, q[:rows], out=out[:rows])
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - min(free) < 8 << 20, [free[0] - f for f in free]

@@ -1339,7 +1339,9 @@ int prefill_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState
         }
     }
     if (int rc = put(c, c->d_pre, host.data(), host.size(), "KVCache prefill batch")) return rc;
-    const size_t ws = zk_paged_prefill_workspace_size(n, total_rows, num_heads, (int)H);
+    // the partials of any batch at once: a small one may need more than a large
+    // one, and growing waits for the device
+    const size_t ws = std::max(zk::kPrefillPartials, zk_paged_prefill_workspace_size(n, total_rows, num_heads, (int)H));
     if (int rc = c->d_pws.ensure(ws, "KVCache prefill workspace")) return rc;
     char *d = (char *)c->d_pre.dev.p;
     const float *dks = fp8 ? (const float *)(d + tbl_bytes + off_bytes + 2 * i32_bytes) : nullptr;

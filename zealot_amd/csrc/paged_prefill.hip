@@ -998,6 +998,8 @@ bool planless(int64_t items, int pages, int64_t fill) {
     return items <= fill || (fill == kFill && items <= 3 * kFill && items * (pages / 2) <= 100000);
 }
 constexpr size_t kPartBytes = (size_t)kRows * (sizeof(float2) + 128 * sizeof(float));  // an item split's partials, D <= 128
+// (slots are at most twice the items, and items x splits at most kFill)
+static_assert(zk::kPrefillPartials == 2 * kFill * kPartBytes, "the most partials");
 
 int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, zk_dtype kv_dtype,
                  void *out, const int32_t *block_tables, const int64_t *cu_seqlens_q, const int64_t *q_off,

@@ -195,6 +195,10 @@ int noalloc_scratch(void **out);
 bool paged_decode_shares_prefixes(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
 // Longest block table (pages per sequence) paged_prefill accepts.
 constexpr int kPrefillMaxPages = 2048;
+// The most that the partials of a planless prefill take (at most 1024 splits of
+// items of 128 rows of (m, l) and 128 floats): any batch's workspace is this or
+// its plan's, whichever is larger.
+constexpr size_t kPrefillPartials = 1024 * 128 * (sizeof(float2) + 128 * sizeof(float));
 // Whether paged_prefill / paged_prefill_rows run this shape (the MFMA kernel's
 // shapes: bf16 or fp8 pools, block_size 16, head_dim 64 or 128, H/Hkv in {1,2,4,8}).
 bool paged_prefill_supported(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
