@@ -30,3 +30,12 @@ def test_scales_match_numpy(D, dtype, off):
         m = np.nanmax(a[cu[n]:cu[n + 1]], axis=(0, 2)) if length else np.zeros(hkv, np.float32)
         want = np.where(m > 0, m.astype(np.float32) / np.float32(448.0), np.float32(1.0))
         np.testing.assert_array_equal(got[n], want)
+
+
+def test_trailing_dimensions_of_one():
+    """x may carry dimensions of one behind [T, Hkv, D]; no sequences, no scales."""
+    from zealot_amd import ops
+    x = torch.randn((900, 2, 64), generator=torch.Generator().manual_seed(1)).cuda()
+    cu = torch.tensor([0, 300, 900], device="cuda")
+    assert torch.equal(ops.fp8_scales(x.unsqueeze(-1), cu), ops.fp8_scales(x, cu))
+    assert ops.fp8_scales(x, cu[:1]).shape == (0, 2)

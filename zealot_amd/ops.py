@@ -85,7 +85,7 @@ def append(k_pool, v_pool, k, v, slot_mapping, k_scales=None, v_scales=None, tok
 def fp8_scales(x, cu_seqlens, stream=None) -> torch.Tensor:
     """Per-(sequence, kv_head) scales amax/448 over x[cu[n]:cu[n+1]] ([T, Hkv, D])."""
     n = cu_seqlens.shape[0] - 1
-    tokens, hkv, d = x.shape
+    tokens, hkv, d = x.shape[0], x.shape[1], x.shape[2]
     out = torch.empty((n, hkv), dtype=torch.float32, device=x.device)
     # parts of at least 64 tokens on average, up to two workgroups a CU: below,
     # the second launch costs more than the parts give.  (Not on a stream of the
