@@ -2,6 +2,8 @@
 of ragged 16-byte chunks, empty and one-token sequences, more chunks than one
 round of a workgroup's loads, all-zero heads (scale 1), NaN (ignored) and
 infinities, and a source off its 16-byte alignment."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -39,3 +41,22 @@ def test_trailing_dimensions_of_one():
     cu = torch.tensor([0, 300, 900], device="cuda")
     assert torch.equal(ops.fp8_scales(x.unsqueeze(-1), cu), ops.fp8_scales(x, cu))
     assert ops.fp8_scales(x, cu[:1]).shape == (0, 2)
+
+
+@pytest.mark.parametrize("n,tokens,want", [(8, 512, 0), (8, 2000, 1), (1, 700, 0), (1, 4000, 1)])
+def test_short_prompts_take_one_launch(n, tokens, want):
+    """Only prompts long enough to gain from parts pay for the launch that merges them."""
+    from zealot_amd import _lib, ops
+    x = torch.randn((n * tokens, 8, 128), device="cuda").bfloat16()
+    cu = (torch.arange(n + 1) * tokens).cuda()
+    lib, launches, ms = _lib.lib(), ctypes.c_int64(), ctypes.c_double()
+    lib.zk_timing_reset()
+    lib.zk_timing_enable(1)
+    got = ops.fp8_scales(x, cu)
+    torch.cuda.synchronize()
+    lib.zk_timing_enable(0)
+    _lib.check(lib.zk_timing_query(b"fp8_scales_merge", ctypes.byref(launches), ctypes.byref(ms)))
+    lib.zk_timing_reset()
+    assert launches.value == want
+    amax = x.view(n, tokens, 8, 128).abs().amax((1, 3)).float().cpu().numpy()
+    np.testing.assert_array_equal(got.cpu().numpy(), amax / np.float32(448.0))

@@ -87,10 +87,13 @@ def fp8_scales(x, cu_seqlens, stream=None) -> torch.Tensor:
     n = cu_seqlens.shape[0] - 1
     tokens, hkv, d = x.shape[0], x.shape[1], x.shape[2]
     out = torch.empty((n, hkv), dtype=torch.float32, device=x.device)
-    # parts of at least 64 tokens on average, up to two workgroups a CU: below,
-    # the second launch costs more than the parts give.  (Not on a stream of the
-    # caller's choice: the scratch belongs to the current one.)
-    parts = min(512 // max(1, n * hkv), tokens // (64 * max(1, n))) if stream is None else 1
+    # Parts of at least 64 tokens on average, up to two workgroups a CU, from 192 KB
+    # a sequence and head on: below, the second launch and the scratch cost more
+    # than the parts give (a call in parts is 11.7 us, most of it the host's; 8
+    # heads of 128 bf16 undivided: 8 x 512 tokens 6.5 us, 8 x 1000 9.5, 8 x 2000 16.7).
+    # (Not on a stream of the caller's choice: the scratch belongs to the current one.)
+    split = stream is None and tokens * d * x.element_size() >= max(1, n) * (192 << 10)
+    parts = min(512 // max(1, n * hkv), tokens // (64 * max(1, n))) if split else 1
     scratch = torch.empty(parts * n * hkv, dtype=torch.float32, device=x.device) if parts > 1 else None
     _lib.check(_lib.lib().zk_fp8_scales_parts(
         _dev(x, "x"), zk_dtype(x), _dev(cu_seqlens, "cu_seqlens", torch.int64), n, hkv, d, out.data_ptr(),
