@@ -71,17 +71,28 @@ def _alloc(vgprs: int) -> int:
 
 
 def _one(regs: dict, needle: str):
-    hits = [v for k, v in regs.items() if needle in k]
+    hits = [k for k in regs if needle in k]
+    assert len(hits) == 1, f"{needle}: {hits}"
+    return regs[hits[0]]
+
+
+def _all(regs: dict, needle: str) -> dict:
+    hits = {k: v for k, v in regs.items() if needle in k}
     assert hits, f"no kernel matching {needle}"
-    return hits[0]
+    return hits
+
+
+# template arguments: cache type (0 f32, 1 bf16, 2 fp8), head size, heads a
+# kv-head, planless, and for the decode row groups and shared prefixes
+MIXED_DECODE = "decode_mfma_kernelILi1ELi128ELi4ELb0ELb0ELb0E"  # the mixed step's: bf16, planned
 
 
 def test_plan_kernels_fit_beside_attention_waves(tmp_path):
     dec = kernel_registers("paged_decode.o", tmp_path)
     pre = kernel_registers("paged_prefill.o", tmp_path)
-    plan = _one(dec, "plan_kernelENS_6Params")
+    plan = _one(dec, "11plan_kernelENS_6Params")
     pplan = _one(pre, "prefill_plan_kernel")
-    decode = _one(dec, "decode_mfma_kernelILi1ELi128ELi4E")  # bf16, D = 128, G = 4: the mixed step's decode
+    decode = _one(dec, MIXED_DECODE)
     for name, (v, a, priv) in (("plan_kernel", plan), ("prefill_plan_kernel", pplan)):
         assert v + a <= 64, f"{name}: {v} VGPRs + {a} AGPRs a lane (at most 64)"
         assert priv == 0, f"{name} spills {priv} bytes a lane"
@@ -91,13 +102,19 @@ def test_plan_kernels_fit_beside_attention_waves(tmp_path):
 
 def test_attention_kernels_register_budgets(tmp_path):
     """The prefill kernel runs two waves a SIMD (two four-wave workgroups a
-    CU), so a wave holds at most 256 registers; the decode kernel one wave a
-    SIMD.  In a mixed step a prefill wave and a decode wave may share a SIMD.
-    Neither kernel spills."""
+    CU), so a wave holds at most 256 registers; the planned decode kernel one
+    wave a SIMD, the planless one two and more where LDS allows (20 KB a wave
+    and less: everything but f32 at a head size of 128).  In a mixed step a
+    prefill wave and a decode wave may share a SIMD.  No instantiation of
+    either kernel spills."""
     dec = kernel_registers("paged_decode.o", tmp_path)
     pre = kernel_registers("paged_prefill.o", tmp_path)
-    decode = _one(dec, "decode_mfma_kernelILi1ELi128ELi4E")
-    prefill = _one(pre, "prefill_mfma_kernelILi1ELi128ELi4E")
-    assert _alloc(prefill[0] + prefill[1]) <= SIMD_VGPRS // 2
-    assert _alloc(decode[0] + decode[1]) + _alloc(prefill[0] + prefill[1]) <= SIMD_VGPRS
-    assert decode[2] == 0 and prefill[2] == 0, "attention kernels must not spill"
+    attention = {**_all(dec, "decode_mfma_kernel"), **_all(pre, "prefill_mfma_kernel")}
+    for name, (v, a, priv) in attention.items():
+        assert priv == 0, f"{name} spills {priv} bytes a lane"
+        one_wave = "decode_mfma_kernelILi0ELi128E" in name
+        assert _alloc(v + a) <= (SIMD_VGPRS if one_wave else SIMD_VGPRS // 2), f"{name}: {v} + {a}"
+    decode = _one(dec, MIXED_DECODE)
+    for planless in (0, 1):
+        prefill = _one(pre, f"prefill_mfma_kernelILi1ELi128ELi4ELb{planless}E")
+        assert _alloc(decode[0] + decode[1]) + _alloc(prefill[0] + prefill[1]) <= SIMD_VGPRS
