@@ -64,7 +64,7 @@ def test_c1_fp32_mha_d32():
     (32, 8, 64, oracle.BF16),    # D=64
     (24, 8, 96, oracle.BF16),    # D=96 -> generic kernel
     (48, 4, 128, oracle.BF16),   # G=12 -> generic kernel
-    (32, 8, 128, oracle.F32),    # fp32 GQA -> generic kernel
+    (32, 8, 128, oracle.F32),    # fp32 GQA on the f32 MFMA
     (4, 4, 256, oracle.F32),     # D=256
 ])
 def test_head_shapes(H, Hkv, D, dt):
@@ -112,7 +112,7 @@ def test_random_batches_against_oracle(seed):
     Hkv = int(rng.choice([1, 2, 4, 8]))
     H = G * Hkv
     D = int(rng.choice([64, 128]))
-    dt = oracle.F32 if seed % 4 == 3 else oracle.BF16  # fp32 pools take the generic kernel
+    dt = oracle.F32 if seed % 4 == 3 else oracle.BF16  # fp32 pools: the f32 MFMA
     mapping = "grouped" if rng.random() < 0.7 else "modulo"
     N = int(rng.integers(1, 49))
     edges = [0, 1, 15, 16, 17, 255, 256, 257, 767, 768, 769]

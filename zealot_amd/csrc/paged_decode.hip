@@ -428,8 +428,8 @@ struct LdsVec<4> { typedef uint32_t T; };
 // over 16 lanes; the scores' fragment is P^T's, as above.  64 MFMAs of 32 cycles
 // a page are 0.85 us, hidden behind the 2.3 us that a page takes at the HBM rate
 // with one wave a SIMD.  48 x 128..4096 tokens, 32 / 8 heads of 128: 2500 us in
-// decode_generic_kernel (a row per lane: uncoalesced, serial), 158 us here
-// (5.5 TB/s).
+// decode_generic_kernel (a row per lane: uncoalesced, serial), 155 us here
+// (5.6 TB/s).
 // DIRECT: no plan and no queue; workgroup (kvh, part, n) is partition `part` of
 // sequence n (at most kDirectPages pages), derives its pages from the length
 // and the table itself and ends.  A partition whose pages end at an invalid
@@ -442,7 +442,8 @@ struct LdsVec<4> { typedef uint32_t T; };
 // 32 cycles a page, 1.7 us, against 0.85 for one row tile).  A 150-token chunk
 // behind 0..600 tokens, 32 / 8 heads of 128: 57 us as 150 one-row decodes, 31
 // here, and its tables no longer displace the decode half's (four uploads of a
-// step gone): the step of it and 12 decodes 113 -> 60 us.
+// step gone): the step of it and 12 decodes 113 -> 59 us.  Pages with tokens that
+// only some of the rows see come last (SOME below).
 // SHARED (with DIRECT): the first num_sg * shared_parts workgroups of a kv-head
 // are the shared-prefix partitions, the others the sequences' own.
 template <int KV, int D, int G, bool DIRECT, bool ROWS = false, bool SHARED = false>
@@ -579,21 +580,21 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
             }
             return;
         } else {
-        const size_t qb = qr * (size_t)p.q_stride + (size_t)qh * D + (size_t)grp * DG;
-        if (p.q_f32) {
-            const float *qq = (const float *)p.q + qb;
+            const size_t qb = qr * (size_t)p.q_stride + (size_t)qh * D + (size_t)grp * DG;
+            if (p.q_f32) {
+                const float *qq = (const float *)p.q + qb;
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                u32x4 w;
+                for (int kk = 0; kk < KK; ++kk) {
+                    u32x4 w;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(qq[8 * kk + 2 * j], qq[8 * kk + 2 * j + 1]);
-                qf[kk] = __builtin_bit_cast(bf16x8, w);
+                    for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(qq[8 * kk + 2 * j], qq[8 * kk + 2 * j + 1]);
+                    qf[kk] = __builtin_bit_cast(bf16x8, w);
+                }
+            } else {
+                const uint16_t *qq = (const uint16_t *)p.q + qb;
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8 *>(qq + 8 * kk);
             }
-        } else {
-            const uint16_t *qq = (const uint16_t *)p.q + qb;
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8 *>(qq + 8 * kk);
-        }
         }
     };
 
@@ -742,19 +743,19 @@ __global__ void __launch_bounds__(kWave) decode_mfma_kernel(Params p) {
                 for (int t = 0; t < T; ++t) sacc[t] += s2[t];
             } else {
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                u32x4 w;
-                if constexpr (KV == ZK_BF16) {
-                    w = u32x4{kw[4 * kk], kw[4 * kk + 1], kw[4 * kk + 2], kw[4 * kk + 3]};
-                } else {
-                    const u32x2 lo2 = e4m3x4_to_bf16x4(kw[2 * kk]), hi2 = e4m3x4_to_bf16x4(kw[2 * kk + 1]);
-                    w = u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
-                }
+                for (int kk = 0; kk < KK; ++kk) {
+                    u32x4 w;
+                    if constexpr (KV == ZK_BF16) {
+                        w = u32x4{kw[4 * kk], kw[4 * kk + 1], kw[4 * kk + 2], kw[4 * kk + 3]};
+                    } else {
+                        const u32x2 lo2 = e4m3x4_to_bf16x4(kw[2 * kk]), hi2 = e4m3x4_to_bf16x4(kw[2 * kk + 1]);
+                        w = u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
+                    }
 #pragma unroll
-                for (int t = 0; t < T; ++t)
-                    sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), qf[t][kk],
-                                                                      sacc[t], 0, 0, 0);
-            }
+                    for (int t = 0; t < T; ++t)
+                        sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), qf[t][kk],
+                                                                          sacc[t], 0, 0, 0);
+                }
             }
             // V rows as bf16 pairs: w[i][j] = dims (2j, 2j+1) of token row
             // 4*grp+i; f32: the DT values themselves
@@ -1785,9 +1786,9 @@ double direct_limit(int kv_dtype, int plan_launches) {
 // kv-heads (each streams its pages for up to 32 rows, beside the sequences' own
 // one- and two-page items, all resident at once), of at least 10 pages.  Against
 // the planned launch (eight queues, 32-page items), four layers of a step, us: 16
-// x 8 forks of 2050 tokens 152 / 139, 12 x 8 of 3900 187 / 172, 5 x 11 of 2420 117 /
-// 107, 8 x 2 of 700 76 / 62, 1 x 2 of 400 70 / 45; 256, 512, 640 and 1024 items 171,
-// 146, 147 and 161 on the first.  Over 8 layers with one plan, us a layer: 8 x 8 of
+// x 8 forks of 2050 tokens 152 / 139 (134 with the merge a kv-head), 12 x 8 of 3900
+// 187 / 172, 5 x 11 of 2420 117 / 107, 8 x 2 of 700 76 / 62, 1 x 2 of 400 70 / 45;
+// 256, 512, 640 and 1024 items 171, 146, 147 and 161 on the first.  Over 8 layers with one plan, us a layer: 8 x 8 of
 // 4000 (131 MB of shared pages) 40.5 / 36, 24 x 8 of 4000 (393) 97 / 97, 16 x 8 of
 // 8000 (525) 125 / 132, 8 x 8 of 16000 (523) 121 / 130, 200 x 4 of 1000 (817) 196 / 211.
 constexpr long kSharedItems = 384, kSharedMinPages = 10;

@@ -413,7 +413,7 @@ prefill_mfma_kernel(PParams p) {
         }
         const int pos0 = p0 * BS;  // positions below are relative to the split
 
-        // rows: column col of this wave's tile t is item row r = 64 w + 16 t + col
+        // rows: column col of this wave's tile t is item row r = 32 w + 16 t + col
         // = token r / G, head r % G
         bf16x8 qf[T][KK];
         int lim[T];       // keys at positions < lim[t] are visible to this lane's row
@@ -791,7 +791,7 @@ prefill_mfma_kernel(PParams p) {
         }
         for (; j < npair; ++j) iter.template operator()<false, 0>(j);
 
-        // rows of this lane: item row 64 w + 16 t + col, dims 16 dt + 4 grp + i
+        // rows of this lane: item row 32 w + 16 t + col, dims 16 dt + 4 grp + i
         // (bf16 pools, transposed V reads) or DT (4 grp + i) + dt (fp8 pools)
 #pragma unroll
         for (int t = 0; t < T; ++t) {
