@@ -77,7 +77,7 @@ struct Plan {
 // of k, and with it another rounding, from timings 1.5 % apart.  The first m of a
 // count that a process meets decides for its others: over m = 1..64 of seven
 // Llama-3-8B products, smallest or largest first, the shared choice takes what a
-// choice an m takes, within what two timings of one m differ by (5 %).
+// choice an m takes, within what two timings of one m draw.
 struct Choice {
     int splits, tile_rows, fused_splits, fused_rows;
     hipblasLtMatmulAlgo_t algo;

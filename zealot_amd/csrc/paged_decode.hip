@@ -1788,9 +1788,11 @@ double direct_limit(int kv_dtype, int plan_launches) {
 // the planned launch (eight queues, 32-page items), four layers of a step, us: 16
 // x 8 forks of 2050 tokens 152 / 139 (134 with the merge a kv-head), 12 x 8 of 3900
 // 187 / 172, 5 x 11 of 2420 117 / 107, 8 x 2 of 700 76 / 62, 1 x 2 of 400 70 / 45;
-// 256, 512, 640 and 1024 items 171, 146, 147 and 161 on the first.  Over 8 layers with one plan, us a layer: 8 x 8 of
-// 4000 (131 MB of shared pages) 40.5 / 36, 24 x 8 of 4000 (393) 97 / 97, 16 x 8 of
-// 8000 (525) 125 / 132, 8 x 8 of 16000 (523) 121 / 130, 200 x 4 of 1000 (817) 196 / 211.
+// 256, 512, 640 and 1024 items 171, 146, 147 and 161 on the first.  Over 8 layers
+// with one plan, us a layer: 8 x 8 of 4000 (131 MB of shared pages) 40.5 / 36, 24 x
+// 8 of 4000 (393) 97 / 97, 16 x 8 of 8000 (525) 125 / 132, 8 x 8 of 16000 (523) 121 /
+// 130, 200 x 4 of 1000 (817) 196 / 211 (but 4 x 32 of 16000, 1018, whose subgroups
+// read the same pages: 162 / 138).
 constexpr long kSharedItems = 384, kSharedMinPages = 10;
 constexpr double kDirectSharedBytes = 0.45e9;
 int direct_parts(double units, double page_bytes, int max_blocks, double limit = kDirectBytes) {
