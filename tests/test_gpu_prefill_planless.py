@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from tests.gpu_util import as_f32, max_abs_err
+from tests.gpu_util import as_f32, max_abs_err, to_dev, to_host
 from tests.test_gpu_prefill import _case, _run
 
 pytestmark = pytest.mark.gpu
@@ -97,3 +97,18 @@ def test_cache_keeps_its_prefill_workspace():
         torch.cuda.synchronize()
         free.append(torch.cuda.mem_get_info()[0])
     assert free[0] - min(free) < 8 << 20, [free[0] - f for f in free]
+
+
+def test_workspace_without_partials():
+    """A workspace that holds the plan and no partials: the same rows, unsplit."""
+    from zealot_amd import ops
+    H, Hkv, D, starts, chunks = 8, 2, 128, [1500, 40], [33, 5]
+    q, kp, vp, kvdt, bt, cu, _, _ = _case(350, H, Hkv, D, starts, chunks)
+    plan = 256 + 2048 + -(-16 * (-(-sum(chunks) // 32) + len(chunks)) * Hkv // 256) * 256
+    assert ops.prefill_workspace_bytes(len(chunks), sum(chunks), H, Hkv) > plan
+    args = [to_dev(x) for x in (q, kp, vp, bt, cu, np.asarray(starts, np.int32))]
+    out = ops.paged_prefill(*args, workspace=torch.empty(plan, dtype=torch.uint8, device="cuda"))
+    ref = oracle.paged_prefill(as_f32(q, oracle.BF16), kp, vp, kvdt, bt, cu, starts, Hkv, D, 16, np.float32(1 / math.sqrt(D)))
+    assert max_abs_err(as_f32(to_host(out), oracle.BF16), ref) <= 2e-2
+    with pytest.raises(RuntimeError, match="workspace"):
+        ops.paged_prefill(*args, workspace=torch.empty(plan - 256, dtype=torch.uint8, device="cuda"))

@@ -161,6 +161,7 @@ struct zk_kv_cache {
     uint64_t tbl_version = 0;  // bumped whenever d_tbl receives different tables
     CachedBuf d_pre;   // prefill batch tables, row offsets, lengths, starts, scales
     DevBuf d_pws;      // prefill workspace
+    bool no_partials = false;  // the device had no room for the prefill's partials
     DevBuf d_ws;     // decode workspace
     static constexpr int kStages = 16;
     Staging stage[kStages];
@@ -1342,7 +1343,13 @@ int prefill_batch(zk_kv_cache *c, size_t layer, const std::vector<const SeqState
     // the partials of any batch at once: a small one may need more than a large
     // one, and growing waits for the device
     const size_t ws = std::max(zk::kPrefillPartials, zk_paged_prefill_workspace_size(n, total_rows, num_heads, (int)H));
-    if (int rc = c->d_pws.ensure(ws, "KVCache prefill workspace")) return rc;
+    if (c->no_partials || c->d_pws.ensure(ws, "KVCache prefill workspace") != ZK_OK) {
+        // a device that the pools leave full: without partials, items are not split
+        c->no_partials = true;
+        (void)hipGetLastError();
+        const size_t least = zk::paged_prefill_plan_bytes(n, total_rows, num_heads, (int)H);
+        if (int rc = c->d_pws.ensure(least, "KVCache prefill workspace")) return rc;
+    }
     char *d = (char *)c->d_pre.dev.p;
     const float *dks = fp8 ? (const float *)(d + tbl_bytes + off_bytes + 2 * i32_bytes) : nullptr;
     const float *dvs = fp8 ? dks + (size_t)n * H : nullptr;

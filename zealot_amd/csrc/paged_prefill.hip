@@ -1008,13 +1008,13 @@ int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void
                  float scale, int causal, zk_gqa_mapping mapping, const float *k_scales, const float *v_scales,
                  void *workspace, size_t workspace_bytes, void *stream, int64_t q_stride, int max_groups);
 
-size_t plan_bytes(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads) {
+}  // namespace
+
+size_t zk::paged_prefill_plan_bytes(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads) {
     return align256(sizeof(int32_t) * (size_t)num_seqs) + kWorkBytes +
            align256(sizeof(int4) * (size_t)max_items_for(num_seqs, total_q, num_heads, num_kv_heads) *
                     (size_t)num_kv_heads);
 }
-
-}  // namespace
 
 int zk::paged_prefill_rows(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool,
                            zk_dtype kv_dtype, void *out, const int32_t *block_tables, const int64_t *q_off,
@@ -1038,7 +1038,7 @@ size_t zk_paged_prefill_workspace_size(int num_seqs, int64_t total_q, int num_he
     // the plan's, or the planless launch's partials
     const int splits = max_splits_for(planless_items(num_seqs, total_q, num_heads, num_kv_heads), kFill);
     const size_t slots = (size_t)max_items_for(num_seqs, total_q, num_heads, num_kv_heads) * num_kv_heads;
-    return std::max(plan_bytes(num_seqs, total_q, num_heads, num_kv_heads), splits > 1 ? slots * splits * kPartBytes : 0);
+    return std::max(paged_prefill_plan_bytes(num_seqs, total_q, num_heads, num_kv_heads), splits > 1 ? slots * splits * kPartBytes : 0);
 }
 
 int zk_paged_prefill(const void *q, zk_dtype q_dtype, const void *k_pool, const void *v_pool, zk_dtype kv_dtype,
@@ -1090,7 +1090,7 @@ int prefill_impl(const void *q, zk_dtype q_dtype, const void *k_pool, const void
     if (fp8 != (k_scales != nullptr && v_scales != nullptr))
         return set_error(ZK_ERR_INVALID_ARGUMENT,
                          "Internal error: zk_paged_prefill: fp8 pools need k/v scales, other pools none");
-    const size_t need = plan_bytes(num_seqs, total_q, num_heads, num_kv_heads);
+    const size_t need = paged_prefill_plan_bytes(num_seqs, total_q, num_heads, num_kv_heads);
     if (workspace_bytes < need || ((uintptr_t)workspace & 255u))
         return set_error(ZK_ERR_INVALID_ARGUMENT,
                          "Internal error: zk_paged_prefill: workspace too small or not 256-B aligned (need " +

@@ -195,6 +195,9 @@ int noalloc_scratch(void **out);
 bool paged_decode_shares_prefixes(int kv_dtype, int head_dim, int block_size, int num_heads, int num_kv_heads);
 // Longest block table (pages per sequence) paged_prefill accepts.
 constexpr int kPrefillMaxPages = 2048;
+// The workspace that a prefill cannot do without: its plan's.  Less than
+// zk_paged_prefill_workspace_size means that items are not split.
+size_t paged_prefill_plan_bytes(int num_seqs, int64_t total_q, int num_heads, int num_kv_heads);
 // The most that the partials of a planless prefill take (at most 1024 splits of
 // items of 128 rows of (m, l) and 128 floats): any batch's workspace is this or
 // its plan's, whichever is larger.
