@@ -176,7 +176,7 @@ def test_decode_suites_with_planned_launches():
     files = ["test_gpu_planned_launches", "test_gpu_decode_planless", "test_gpu_prefix_planless", "test_gpu_kv_cache", "test_gpu_decode"]
     r = subprocess.run([sys.executable, "-u", "-m", "pytest", "-x", "-q", "-m", "gpu", "-p", "no:cacheprovider", "-k", "not full_size and not prefill",
                         *(os.path.join(here, f + ".py") for f in files)], cwd=os.path.dirname(here), capture_output=True, text=True,
-                       timeout=110, env={**os.environ, "ZEALOT_DECODE_PART_PAGES": "16"})
+                       timeout=170, env={**os.environ, "ZEALOT_DECODE_PART_PAGES": "16"})
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
 
 
